@@ -528,10 +528,14 @@ size_t gemv_scratch_bytes(int sem, int n_rows, int n_cols, int B)
 }
 
 // Queue GEMV(s) over B tokens (any B: split into groups of 8) on device data;
-// out_add (optional, same layout as out, not overlapping it on the MFMA path)
-// is added to the result.
+// out_add (optional, same layout as out; on the bf16-tile GEMM not overlapping
+// it, on the fp16-plane GEMM equal to it or apart) is added to the result.
+// pro (fp16-plane GEMM only): the activation's prologue, formed while it is staged;
+// x then has row stride ldx.  pair (there only, where the launch splits K): n_rows gate
+// and up rows, out = silu(gate) * up of n_rows / 2.
 int run_gemv(int sem, const mllm_packed &W, const float *x, float *out, int n_rows, int n_cols, int B,
-             void *scratch, hipStream_t st, const float *out_add = nullptr, bool gemm_ok = true)
+             void *scratch, hipStream_t st, const float *out_add = nullptr, bool gemm_ok = true,
+             const act16_pro *pro = nullptr, int ldx = 0, bool pair = false, bool clamp = false)
 {
     const bool q8 = mllm_sem_uses_q8(sem);
     if (gemm_ok && uses_q16(sem, n_cols, B)) {
@@ -546,16 +550,17 @@ int run_gemv(int sem, const mllm_packed &W, const float *x, float *out, int n_ro
         }
         const act16 ac = mllm_act16_carve(sem, ws, B, n_cols);
         ws += mllm_act16_bytes(sem, B, n_cols);
-        HIP_OK(mllm_launch_act16(sem, x, n_cols, q8 ? &xq : nullptr, B, n_cols, ac, st));
+        if (pro) HIP_OK(mllm_launch_act16_pro(sem, x, ldx, *pro, B, n_cols, ac, st));
+        else HIP_OK(mllm_launch_act16(sem, x, n_cols, q8 ? &xq : nullptr, B, n_cols, ac, st));
         q16_args g{};
         g.W = W;
         g.x = ac;
-        g.out = out; g.ldo = n_rows;
+        g.out = out; g.ldo = pair ? n_rows / 2 : n_rows;
+        g.add = out_add; g.pair = pair; g.clamp_silu = clamp;
         g.n_rows = n_rows; g.n_cols = n_cols; g.n_entries = B;
         g.ksplit = mllm_q16_ksplit(sem, n_rows, n_cols, B);
         if (g.ksplit > 1) g.part = (float *)ws;
         HIP_OK(mllm_launch_q16(sem, false, g, 0, st));
-        if (out_add) HIP_OK(mllm_launch_add(out, out_add, (long)B * n_rows, st));
         return 0;
     }
     if (gemm_ok && B > 8 && mllm_qgemm_supported(sem) && n_cols >= mllm_sem_block_elems(sem)) {
@@ -1165,7 +1170,16 @@ MLLM_API int mllm_gemv_fused(int sem, const void *packed_dev, const float *x_dev
     }
     uint8_t *ws = (uint8_t *)workspace;
     const float *xa = x_dev;
-    if (f && (pro || f->x_up)) {
+    const bool act = f && (pro || f->x_up);
+    const bool q16 = uses_q16(sem, n_cols, B);
+    // the fp16-plane GEMM forms the activation while it stages it (rows its registers hold,
+    // fp32-activation semantics): at B = 32 x 2048 the separate launch took 6.8 us and staging
+    // 4.1 us, together 5
+    act16_pro p16{};
+    const bool pro16 = act && q16 && !mllm_sem_uses_q8(sem) && n_cols <= kAct16ProMax;
+    if (pro16) {
+        p16 = {f->x_up, f->x_res, f->res_out, f->rms_w, f->rms_eps, f->rms_div, f->silu_clamp};
+    } else if (act) {
         float *xe = (float *)ws;
         HIP_OK(mllm_launch_act_prologue(x_dev, f->x_res, f->res_out, f->rms_w, f->rms_eps, f->rms_div, f->x_up,
                                         f->silu_clamp, B, n_cols, ldx, xe, st));
@@ -1174,19 +1188,28 @@ MLLM_API int mllm_gemv_fused(int sem, const void *packed_dev, const float *x_dev
         set_error("mllm_gemv_fused: a strided x (x_ld) needs a fused activation step on this path");
         return -1;
     }
+    if (pair && q16 && mllm_q16_ksplit(sem, mrows, n_cols, B) > 1)
+        // gate, up and the SiLU product joined from the split's partial sums
+        return run_gemv(sem, view, xa, out_dev, mrows, n_cols, B, ws + L.gemv, st, out_add, true, pro16 ? &p16 : nullptr,
+                        ldx, true, f->silu_clamp != 0);
     if (pair) {
         float *y = (float *)(ws + L.pair);
-        if (run_gemv(sem, view, xa, y, mrows, n_cols, B, ws + L.gemv, st)) return -1;
+        if (run_gemv(sem, view, xa, y, mrows, n_cols, B, ws + L.gemv, st, nullptr, true, pro16 ? &p16 : nullptr, ldx))
+            return -1;
         HIP_OK(mllm_launch_silu_pair(y, B, n_rows, f->silu_clamp, out_dev, out_add, st));
         return 0;
     }
-    if (out_add && B > 8) {
-        // the MFMA path writes out before the residual is added: add from a copy
+    const size_t osz = (size_t)B * n_rows * 4;
+    const uintptr_t ao = (uintptr_t)out_add, oo = (uintptr_t)out_dev;
+    if (out_add && B > 8 && !(q16 && (ao == oo || ao + osz <= oo || oo + osz <= ao))) {
+        // the bf16-tile GEMM writes out before the residual is added: add from a copy (the
+        // fp16-plane GEMM adds where it writes, so it needs one only for a partial overlap)
         float *keep = (float *)(ws + L.keep);
         HIP_OK(hipMemcpyAsync(keep, out_add, (size_t)B * n_rows * 4, hipMemcpyDeviceToDevice, st));
         out_add = keep;
     }
-    return run_gemv(sem, view, xa, out_dev, n_rows, n_cols, B, ws + L.gemv, st, out_add);
+    return run_gemv(sem, view, xa, out_dev, n_rows, n_cols, B, ws + L.gemv, st, out_add, true, pro16 ? &p16 : nullptr,
+                    ldx);
 }
 
 // ------------------------------------------------ lm_head requantisation (f2)

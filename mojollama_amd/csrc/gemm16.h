@@ -74,6 +74,19 @@ act16 mllm_act16_carve(int sem, void *ws, long rows, int K);
 // mllm_launch_quantize_q8_0's quants and min-term sums) -> act.
 hipError_t mllm_launch_act16(int sem, const float *x, int ldx, const mllm_xq *xq, int rows, int K, const act16 &act,
                              hipStream_t st);
+// The activation work before a fused GEMM (mllm_gemv_fusion), done while act16 stages its
+// rows: v = x (silu(x) * x_up) (+ x_res), res_out = v, v * rms / norm weights.  All of the
+// row stays in registers between the passes, so rows of at most kAct16ProMax elements.
+struct act16_pro {
+    const float *x_up, *x_res;
+    float *res_out;
+    const float *rms_w;
+    float rms_eps;
+    int rms_div, silu_clamp;
+};
+constexpr int kAct16ProMax = 8192;
+hipError_t mllm_launch_act16_pro(int sem, const float *x, int ldx, const act16_pro &pro, int rows, int K,
+                                 const act16 &act, hipStream_t st);
 
 // out[out_row(p)][n] = W[n] . x[row_of(p)] over the entries p of each work
 // tile: the consecutive slices of [0, n_entries) (tile_expert == nullptr), or
@@ -95,6 +108,11 @@ struct q16_args {
     int clamp_silu;
     int ksplit;
     float *part;
+    // dense launches: out = add + W x (add: out's layout; may be out itself).  pair: the matrix
+    // holds gate rows then up rows, n_rows in all; out[e][r] (r < n_rows / 2) = silu(gate) * up,
+    // the gate clamped when clamp_silu; formed from the partial sums, so ksplit > 1 only
+    const float *add;
+    int pair;
     int eoff;        // MXFP4: weights decode as v 2^(E + eoff) (mllm_q16_mx_shift)
     float wscale;    // MXFP4: 2^(-127 - eoff), applied to the result
     int rows_fast;   // set by the launch: work tiles ordered row block fastest

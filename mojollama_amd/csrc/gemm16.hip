@@ -860,6 +860,12 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
                 }
                 v[r] = x0;
             }
+            if (a.add && a.ksplit <= 1) {   // the residual, read by the lane that writes its place
+                const float *ad = a.add + orow * ldo + n;
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (n + r < a.n_rows) v[r] = ad[r] + v[r];
+            }
             if (n + 3 < a.n_rows && (ldo & 3) == 0) {
                 *reinterpret_cast<float4 *>(o + n) = make_float4(v[0], v[1], v[2], v[3]);
             } else {
@@ -871,16 +877,58 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
     }
 }
 
-// out[e][n] = sum over z < ks of part[z][e][n], in order.
-__global__ void k_q16_ksum(const float *__restrict__ part, int ks, long plane, int n_rows, float *__restrict__ out,
-                           int ldo)
+// The split-K partial sums joined, in order: out[e][n] = sum over z < ks of part[z][e][n]
+// (+ add).  PAIR: part rows hold n_out gate sums, then n_out up sums; out = silu(g) * u
+// (+ add).  V consecutive outputs a thread (4 where every row is a multiple of 4 floats),
+// so a thread has ks (2 ks) 16-byte loads in flight.  One launch for what were three (join,
+// residual add after a copy of the residual, SiLU product): at 32 tokens each of those is a
+// launch of 4 to 5 us that moves under 1 MB.
+template <bool PAIR, int V>
+__global__ __launch_bounds__(256) void k_q16_join(const float *__restrict__ part, int ks, long plane, int n_out,
+                                                  int n_ent, float *out, int ldo, const float *add, int clamp)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= plane) return;
-    float v = part[i];
-    for (int z = 1; z < ks; z++) v += part[z * plane + i];
-    const long e = i / n_rows, n = i - e * n_rows;
-    out[e * ldo + n] = v;
+    const int per = n_out / V;
+    if (i >= (long)per * n_ent) return;
+    const long e = i / per;
+    const int n = (int)(i - e * per) * V;
+    const float *p = part + e * (PAIR ? 2 * n_out : n_out) + n;
+    float g[V], u[V];
+    auto ld = [&](const float *q, float (&v)[V]) __attribute__((always_inline)) {
+        if constexpr (V == 4) {
+            const float4 w = *reinterpret_cast<const float4 *>(q);
+            v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
+        } else {
+            v[0] = *q;
+        }
+    };
+    ld(p, g);
+    if constexpr (PAIR) ld(p + n_out, u);
+#pragma unroll 4
+    for (int z = 1; z < ks; z++) {
+        float t[V];
+        ld(p + z * plane, t);
+#pragma unroll
+        for (int k = 0; k < V; k++) g[k] += t[k];
+        if constexpr (PAIR) {
+            ld(p + z * plane + n_out, t);
+#pragma unroll
+            for (int k = 0; k < V; k++) u[k] += t[k];
+        }
+    }
+    float *o = out + e * ldo + n;
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int k = 0; k < V; k++) g[k] = mllm_silu_mul(g[k], u[k], clamp != 0);
+    }
+    if (add) {
+        float t[V];
+        ld(add + e * ldo + n, t);
+#pragma unroll
+        for (int k = 0; k < V; k++) g[k] = t[k] + g[k];
+    }
+    if constexpr (V == 4) *reinterpret_cast<float4 *>(o) = make_float4(g[0], g[1], g[2], g[3]);
+    else *o = g[0];
 }
 
 // ---------------------------------------------------------------- activations
@@ -889,15 +937,17 @@ __global__ void k_q16_ksum(const float *__restrict__ part, int ks, long plane, i
 // sub-block.  One workgroup per row.  MXFP4 x Q8_0 first quantises the row to
 // Q8_0 and takes quant times block scale (int8 times an fp16 value: exact in
 // fp32), the activation mxfp4_row_dot_q8 (QK:629-678) multiplies.
-template <int SEM, int TPR>
-__global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int ldx, int K, int rows, act16 a)
+// PRO: the row's prologue (act16_pro) first, on the values held in registers.
+template <int SEM, int TPR, bool PRO>
+__global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int ldx, int K, int rows, act16 a,
+                                               act16_pro pro)
 {
     using Q = q16_traits<SEM>;
     // TPR threads per row: the workgroup (256), or a wave (64) for short rows (at most
     // kHeld * 512 positions), four rows per workgroup and no barrier
     static_assert(TPR == 256 || TPR == 64, "a workgroup or a wave per row");
     constexpr int STR = 8 * TPR;   // positions per iteration
-    __shared__ float red[4];
+    __shared__ float red[4], red_ss[4];
     const int tid = threadIdx.x, lt = tid % TPR;
     const int row = blockIdx.x * (256 / TPR) + tid / TPR;
     if (blockIdx.x == gridDim.x - 1) {   // the last workgroup: the zero row
@@ -963,16 +1013,68 @@ __global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int 
         for (int j = 0; j < 8; j++)
             if (fabsf(v[j]) < INFINITY) m = fmaxf(m, fabsf(v[j]));
     };
+    float ss = 0.0f;   // PRO: the row's sum of squares
 #pragma unroll
     for (int it = 0; it < kHeld; it++)
         if (it < nit) {
-            ld8(gbase(8 * lt + STR * it), g[it]);
-            mx(g[it]);
+            const int k = gbase(8 * lt + STR * it);
+            ld8(k, g[it]);
+            if constexpr (PRO) {
+                const long xo = (long)row * ldx + k;
+                float t[8];
+                auto ld = [&](const float *q) __attribute__((always_inline)) {
+                    if (vec) {
+                        const float4 b = *reinterpret_cast<const float4 *>(q), c = *reinterpret_cast<const float4 *>(q + 4);
+                        t[0] = b.x; t[1] = b.y; t[2] = b.z; t[3] = b.w; t[4] = c.x; t[5] = c.y; t[6] = c.z; t[7] = c.w;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 8; j++) t[j] = q[j];
+                    }
+                };
+                if (pro.x_up) {
+                    ld(pro.x_up + xo);
+#pragma unroll
+                    for (int j = 0; j < 8; j++) g[it][j] = mllm_silu_mul(g[it][j], t[j], pro.silu_clamp != 0);
+                }
+                if (pro.x_res) {
+                    ld(pro.x_res + xo);
+#pragma unroll
+                    for (int j = 0; j < 8; j++) g[it][j] += t[j];
+                }
+                if (pro.res_out) {
+#pragma unroll
+                    for (int j = 0; j < 8; j++) pro.res_out[xo + j] = g[it][j];
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++) ss = fmaf(g[it][j], g[it][j], ss);
+            }
+            if (!PRO || !pro.rms_w) mx(g[it]);
         }
-    for (int it = kHeld; it < nit; it++) {
-        float v[8];
-        ld8(gbase(8 * lt + STR * it), v);
-        mx(v);
+    if constexpr (PRO) {
+        if (pro.rms_w) {
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+            if constexpr (TPR == 256) {
+                if ((tid & 63) == 0) red_ss[tid >> 6] = ss;
+                __syncthreads();
+                ss = red_ss[0] + red_ss[1] + red_ss[2] + red_ss[3];
+            }
+            const float r = sqrtf(ss / (float)K + pro.rms_eps), sc = pro.rms_div ? r : 1.0f / r;
+#pragma unroll
+            for (int it = 0; it < kHeld; it++)
+                if (it < nit) {
+                    const float *w = pro.rms_w + gbase(8 * lt + STR * it);
+#pragma unroll
+                    for (int j = 0; j < 8; j++) g[it][j] = (pro.rms_div ? g[it][j] / sc : g[it][j] * sc) * w[j];
+                    mx(g[it]);
+                }
+        }
+    } else {
+        for (int it = kHeld; it < nit; it++) {
+            float v[8];
+            ld8(gbase(8 * lt + STR * it), v);
+            mx(v);
+        }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
@@ -1025,12 +1127,13 @@ __global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int 
 #pragma unroll
     for (int it = 0; it < kHeld; it++)
         if (it < nit) emit(8 * lt + STR * it, g[it], held1[it]);
-    for (int it = kHeld; it < nit; it++) {
-        float v[8];
-        f16x8 v1;
-        ld8(gbase(8 * lt + STR * it), v);
-        emit(8 * lt + STR * it, v, v1);
-    }
+    if constexpr (!PRO)
+        for (int it = kHeld; it < nit; it++) {
+            float v[8];
+            f16x8 v1;
+            ld8(gbase(8 * lt + STR * it), v);
+            emit(8 * lt + STR * it, v, v1);
+        }
     if constexpr (Q::GGML) {
         for (int j = nb * 8 + lt; j < a.ldm; j += TPR) {
             a.m[(long)row * a.ldm + j] = (_Float16)0.0f;
@@ -1163,8 +1266,17 @@ hipError_t launch16(const q16_args &a, int max_tiles, hipStream_t st)
     hipLaunchKernelGGL((k_q16<SEM, DUAL, EB, SM>), grid, dim3(2 * TN), 0, st, b);
     if (ks > 1) {
         const long plane = (long)a.n_entries * a.n_rows;
-        hipLaunchKernelGGL(k_q16_ksum, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0, st, a.part, ks, plane,
-                           a.n_rows, a.out, a.ldo);
+        const int n_out = a.pair ? a.n_rows / 2 : a.n_rows;
+        const bool v4 = n_out % 4 == 0 && a.ldo % 4 == 0 &&
+                        (((uintptr_t)a.out | (uintptr_t)a.part | (uintptr_t)a.add) & 15) == 0;
+        const long n = (long)a.n_entries * (n_out / (v4 ? 4 : 1));
+        const dim3 g((unsigned)((n + 255) / 256));
+        auto go = [&](auto pair_c, auto v_c) {
+            hipLaunchKernelGGL((k_q16_join<decltype(pair_c)::value, decltype(v_c)::value>), g, dim3(256), 0, st,
+                               a.part, ks, plane, n_out, a.n_entries, a.out, a.ldo, a.add, a.clamp_silu);
+        };
+        if (a.pair) v4 ? go(std::true_type{}, std::integral_constant<int, 4>{}) : go(std::true_type{}, std::integral_constant<int, 1>{});
+        else v4 ? go(std::false_type{}, std::integral_constant<int, 4>{}) : go(std::false_type{}, std::integral_constant<int, 1>{});
     }
     return hipGetLastError();
 }
@@ -1289,9 +1401,9 @@ hipError_t mllm_launch_act16(int sem, const float *x, int ldx, const mllm_xq *xq
     auto go = [&](auto sem_c) {
         constexpr int S = decltype(sem_c)::value;
         if (wave)
-            hipLaunchKernelGGL((k_act16<S, 64>), dim3((rows + 3) / 4 + 1), dim3(256), 0, st, x, ldx, K, rows, act);
+            hipLaunchKernelGGL((k_act16<S, 64, false>), dim3((rows + 3) / 4 + 1), dim3(256), 0, st, x, ldx, K, rows, act, act16_pro{});
         else
-            hipLaunchKernelGGL((k_act16<S, 256>), dim3(rows + 1), dim3(256), 0, st, x, ldx, K, rows, act);
+            hipLaunchKernelGGL((k_act16<S, 256, false>), dim3(rows + 1), dim3(256), 0, st, x, ldx, K, rows, act, act16_pro{});
     };
     switch (sem) {
     case SEM_Q4_K_GGML: go(std::integral_constant<int, SEM_Q4_K_GGML>{}); break;
@@ -1308,12 +1420,36 @@ hipError_t mllm_launch_act16(int sem, const float *x, int ldx, const mllm_xq *xq
     return hipGetLastError();
 }
 
+hipError_t mllm_launch_act16_pro(int sem, const float *x, int ldx, const act16_pro &pro, int rows, int K,
+                                 const act16 &act, hipStream_t st)
+{
+    if (rows <= 0) return hipSuccess;
+    if (K < 256 || K % 256 || K > kAct16ProMax || ((uintptr_t)act.h & 15)) return hipErrorInvalidValue;
+    // a workgroup per row whatever its length: the rows are few (B tokens) and their latency counts
+    const dim3 g(rows + 1);
+#define PRO16(S) case S: hipLaunchKernelGGL((k_act16<S, 256, true>), g, dim3(256), 0, st, x, ldx, K, rows, act, pro); break;
+    switch (sem) {
+    PRO16(SEM_Q4_K_GGML)
+    PRO16(SEM_Q6_K_SEQ)
+    PRO16(SEM_Q6_K_LOWNIB)
+    default: return hipErrorInvalidValue;
+    }
+#undef PRO16
+    return hipGetLastError();
+}
+
 // Dense launches take 128-entry tiles once there are 256 entries, else 64;
 // grouped launches the bucketing's 64-entry tiles.
 int mllm_q16_tile_entries(bool grouped, int n_entries) { return !grouped && n_entries >= 256 ? 128 : 64; }
 
 // Split along K (whole super-blocks) while a dense launch has fewer than two
-// tiles per CU (512), each split keeping at least 4 super-blocks.
+// tiles per CU (512), each split keeping at least 4 super-blocks.  Launches of
+// one entry tile (at most 64 tokens) split down to a super-block per workgroup:
+// their time is the chain of a workgroup's steps, not the partial sums' traffic
+// (rows x K at 32 tokens, staging and join included, at least 4 super-blocks
+// each against at least 1: 2560 x 2048 21.7 -> 16.4 us, 2048 x 5632 36.9 ->
+// 23.7; at least 2: 17.8 and 25.2; 768 workgroups for 512: 11264 x 2048 23.0
+// -> 24.5, 32000 x 2048 38.9 -> 46.4).
 int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries)
 {
     if (!mllm_q16_supported(sem) || n_entries <= 0) return 1;   // MXFP4: grouped launches, no split
@@ -1321,6 +1457,7 @@ int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries)
     const long tiles = (long)((n_rows + 127) / 128) * ((n_entries + tm - 1) / tm);
     if (tiles >= 384) return 1;
     const int nb = n_cols / 256;
+    if (n_entries <= 64) return std::max(1, std::min({(int)(512 / tiles), nb, 32}));
     int ks = (int)(512 / tiles);
     ks = std::min(ks, std::max(1, nb / 4));
     return std::max(1, std::min(ks, 8));

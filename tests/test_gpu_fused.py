@@ -174,3 +174,45 @@ def test_fused_silu_pair(dev, orc, sem, C, B, mode):
     err = O.norm_err(got, ref)
     print(f"[parity] fused pair {K.SEM_NAMES[sem]} {R}x{C} B={B} {mode}: {err:.3e}", flush=True)
     assert err < tol, K.last_error(dev.so)
+
+
+@pytest.mark.parametrize("sem,R,C,B", [(K.Q4_K_GGML, 303, 2048, 9), (K.Q6_K_SEQ, 130, 5632, 33),
+                                       (K.Q4_K_GGML, 2048, 256, 64), (K.Q6_K_SEQ, 516, 9216, 11),
+                                       (K.Q4_K_GGML, 4100, 512, 300), (K.Q4_K_Q8, 300, 2048, 40)])
+@pytest.mark.parametrize("mode", ["rms", "rms_div_res", "res_add", "add_inplace", "silu"])
+def test_fused_batched(dev, orc, sem, R, C, B, mode):
+    """B > 8 on the fp16-plane GEMM: the prologue formed while the activation
+    is staged (rows up to 8192; 9216 takes the separate launch), K split down
+    to one super-block per workgroup, the residual added in the join of the
+    partial sums or, unsplit, in the GEMM's own epilogue."""
+    run_case(dev, orc, sem, R, C, B, mode, seed=R + C + B + len(mode))
+
+
+@pytest.mark.parametrize("sem,R,C,B", [(K.Q4_K_GGML, 150, 2048, 9), (K.Q4_K_GGML, 301, 512, 65),
+                                       (K.Q6_K_LOWNIB, 96, 768, 33), (K.Q4_K_Q8, 128, 1024, 17),
+                                       (K.Q4_K_GGML, 24580, 256, 10)])
+@pytest.mark.parametrize("mode", ["pair", "pair_rms", "pair_noclamp_add"])
+def test_fused_silu_pair_batched(dev, orc, sem, R, C, B, mode):
+    """Paired rows at B > 8: the SiLU product in the join of the split's
+    partial sums (rows of 4-float multiples and odd ones), or after the GEMM
+    where the launch does not split (24580 rows)."""
+    QT.setdefault(K.Q6_K_LOWNIB, 14)
+    import torch
+    rng = np.random.default_rng(sem * 7 + C + B + len(mode))
+    w = W.gen_weights(rng, QT[sem], 2 * R, C)
+    x = W.gen_x(rng, B, C)
+    g = (rng.standard_normal(C) * 0.5 + 1.0).astype(np.float32)
+    add = W.gen_x(rng, B, R)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    packed, gt, addt = dev.pack(sem, cu(w), 2 * R, C), cu(g), cu(add)
+    clamp, rms = mode != "pair_noclamp_add", mode == "pair_rms"
+    f = dev.fusion(silu_pair=True, silu_clamp=clamp, rms_w=gt if rms else None, rms_eps=1e-5,
+                   out_add=None if clamp else addt)
+    got = dev.gemv_fused(sem, packed, cu(x), R, C, f).cpu().numpy()
+    xe = rms_np(x, g, 1e-5, False) if rms else x
+    y = orc.gemv(sem, w, np.ascontiguousarray(xe, np.float32), 2 * R, C, B).astype(np.float64)
+    ref = silu_np(y[:, :R], y[:, R:], clamp) + (0 if clamp else add)
+    tol = MOE_Q8H_TOL if mllm_q8(sem) else GEMV_TOL
+    err = O.norm_err(got, ref)
+    print(f"[parity] fused pair {K.SEM_NAMES[sem]} {R}x{C} B={B} {mode}: {err:.3e}", flush=True)
+    assert err < tol, K.last_error(dev.so)
