@@ -261,3 +261,39 @@ def test_rope_vs_oracle(dev, orc, nh, hd, r):
     for t in range(T):
         ref = orc.rope(x[t], nh, hd, pos[t], cos_t, sin_t, r)
         assert np.max(np.abs(got[t] - ref)) <= 1e-6 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("mode", [O.ATTN_CE, O.ATTN_GQA_C])
+@pytest.mark.parametrize("nh,nkh,hd,S_list,page", [
+    (16, 1, 64, [257, 3], 0), (6, 2, 36, [130, 513], 16), (20, 4, 80, [255, 256, 1], 0), (3, 3, 4, [64, 300], 16),
+    (32, 2, 256, [100, 1030], 0), (64, 64, 20, [70] * 40, 0), (14, 2, 128, [190, 700], 64)])
+def test_gqa_decode_edges(dev, orc, mode, nh, nkh, hd, S_list, page):
+    """Head counts, head sizes and lengths at the edges of the kernels' units:
+    groups of 1 to 16 heads (and odd ones), rows that end inside a 16- or
+    32-element block or span several 64-element ones, one group of four chunks
+    or more, both splits of the heads over workgroups; rows past a sequence's
+    end hold NaN and infinities."""
+    import torch
+    if mode == O.ATTN_GQA_C and nh == 64:
+        # 2560 heads: among them one whose weights, of both signs, sum to about 1/2000 of their
+        # magnitudes, where the fp32 rounding of that sum alone (S 2^-24 of the magnitudes) is
+        # 70 * 6e-8 * 2000 = 8e-3 of the output; below eight positions all weights are positive
+        S_list = [6] * len(S_list)
+    rng = np.random.default_rng(sum(S_list) + nh + hd + 7 * mode)
+    B = len(S_list)
+    q, k, v = make_case(rng, B, S_list, nh, nkh, hd)
+    Smax = k.shape[1]
+    for b, S in enumerate(S_list):
+        k[b, S:], v[b, S:] = np.nan, np.inf
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    if page:
+        kp, vp, tables, n_pages = paged_copy(rng, k, v, S_list, page, nkh, hd)
+        kv = dev.kv_view(cu(kp), cu(vp), block_tables=cu(tables), page_size=page, n_pages=n_pages)
+    else:
+        kv = dev.kv_view(cu(k), cu(v), seq_stride=Smax * nkh * hd)
+    lens = torch.tensor(S_list, dtype=torch.int32, device="cuda")
+    got = dev.gqa_decode(mode, cu(q), kv, lens, Smax, nh, nkh, hd).cpu().numpy()
+    for b, S in enumerate(S_list):
+        ref = orc.gqa_decode(mode, q[b], k[b], v[b], S, nh, nkh, hd)
+        err = np.max(np.abs(got[b] - ref))
+        assert err <= attn_tol(orc, mode, q[b], k[b], v[b], S, nh, nkh, hd, ref), (b, S, err, np.max(np.abs(ref)))
