@@ -105,6 +105,7 @@ struct q16_args {
     const int *out_row;
     int n_rows, n_cols, n_entries;
     const int *tile_expert, *tile_begin, *tile_end, *n_tiles;
+    int tile32;      // grouped: the tiles hold at most 32 entries (mllm_q16_tile32), else 64
     int clamp_silu;
     int ksplit;
     float *part;
@@ -122,6 +123,8 @@ struct q16_args {
     const uint8_t *sm, *sm2;
     long sm_stride, sm_doff;
 };
+// Whether a grouped launch can take 32-entry tiles (needs step-major metadata).
+bool mllm_q16_tile32(int sem, bool dual);
 // Entries per work tile of a launch (grouped launches: the bucketing's tile).
 int mllm_q16_tile_entries(bool grouped, int n_entries);
 int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries);

@@ -51,8 +51,10 @@ template <int SEM> struct q16_traits {
 // each activation tile staged in LDS serves twice the rows (the activation loads bound
 // these GEMMs; Qwen3's short-K Q6_K down gained 4%, bit-identical); gate + up, whose
 // two matrices already share each tile, and the 128-entry dense tiles keep 128.
+// 32-entry tiles (EB == 1) have too few entries for eight waves to load.
 template <int SEM, bool DUAL, int EB> constexpr int q16_wpg()
 {
+    if (EB == 1) return 4;
     return (q16_traits<SEM>::MX || (q16_traits<SEM>::Q6 && EB == 2)) && !DUAL ? 8 : 4;
 }
 
@@ -212,11 +214,13 @@ MLLM_DEV void q16_decode_mx(const q16_raw &r, int kh, int eoff, u32x4 (&o)[4])
     }
 }
 
-// v and its fp16 remainder: v = hi + lo (lo the fp16 rounding of v - hi).
+// v and its fp16 remainder: v = hi + lo (lo the fp16 rounding of v - hi; 0 where v is
+// infinite, so that a product with a finite weight stays infinite, and hi is NaN for a NaN).
 MLLM_DEV void split16(float v, _Float16 &hi, _Float16 &lo)
 {
     hi = (_Float16)v;
-    lo = (_Float16)(v - (float)hi);
+    const float r = v - (float)hi;
+    lo = (_Float16)(r == r ? r : 0.0f);
 }
 
 // Q4_K min-term weights of one row for one k16 slice of the min product: 8 values at once.
@@ -316,8 +320,16 @@ template <class T> MLLM_DEV T gldo(const void *base, uint32_t off) { return gld<
 
 // SM: the matrices' super-block metadata (MXFP4: exponents) read from the step-major copy
 // (a.sm, mllm_launch_q16_smeta) instead of the packed planes.
+// EB == 1 (32-entry tiles, few tokens per expert): the launch streams weights, so its rate
+// is the workgroups in flight; half the accumulators and a quarter of the LDS admit three or
+// four per CU where 64-entry tiles have two.
+template <int SEM, bool DUAL, int EB> constexpr int q16_waves()   // per SIMD
+{
+    return EB == 1 ? (DUAL ? 3 : 4) : 8 / q16_wpg<SEM, DUAL, EB>();
+}
+
 template <int SEM, bool DUAL, int EB, bool SM>
-__global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, DUAL, EB>())) void k_q16(q16_args a)
+__global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (q16_waves<SEM, DUAL, EB>())) void k_q16(q16_args a)
 {
     using Q = q16_traits<SEM>;
     constexpr int WPG = q16_wpg<SEM, DUAL, EB>(), RB = DUAL ? 2 : 1, TM = 32 * EB, TN = 32 * WPG, SPB = Q::SPB, NPL = Q::NPL;
@@ -401,8 +413,9 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
     // load instructions per wave, plane and step (four waves: EB; MXFP4's eight: one, for
     // waves whose rows the tile's entry blocks reach)
     constexpr int NCH = TM * 8 / (64 * WPG);
-    constexpr bool B8 = MX;   // K-quant tiles keep four buffers (their LDS then admits a third workgroup per CU)
+    constexpr bool B8 = MX || EB == 1;   // larger K-quant tiles keep four buffers (their LDS then admits a third workgroup per CU)
     constexpr int D2 = B8 ? 3 : 1;      // two-plane prefetch distance (steps)
+    constexpr bool UW = MX && EB == 1 && !DUAL;   // weights fetched a unit (four steps) at a time, see main_loop
     __shared__ __attribute__((aligned(16))) _Float16 sB0[TM * 64], sB1[TM * 64], sB2[TM * 64], sB3[TM * 64];
     __shared__ __attribute__((aligned(16))) _Float16 sB4[B8 ? TM * 64 : 8], sB5[B8 ? TM * 64 : 8],
         sB6[B8 ? TM * 64 : 8], sB7[B8 ? TM * 64 : 8];
@@ -612,7 +625,12 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
         // overstates what may stay in flight, which their own loads never need)
         constexpr int NDMA = WPG == 8 ? NP : NEB * NP;
         const int s_beg = b_beg * SPB, s_last = b_end * SPB - 1;
-        q16_raw rw[4][RB];
+        // UW: a unit's weights are fetched together, one unit ahead (rn: the next unit's).  A row's
+        // bytes of the four steps are one 128-byte line (MXFP4: half a line's nibbles a step pair):
+        // fetched step by step, microseconds apart, the line leaves L1 in between and comes from
+        // L2 four times (GPT-OSS down at 16 tokens: 49.0 -> 43.6 us; the fused gate + up, which
+        // waits on its decode and MFMAs, 90.6 -> 92.4, and the K-quants spill)
+        q16_raw rw[4][RB], rn[UW ? 4 : 1][RB];
         // super-block metadata (Q4_K: kq_pairs layout; Q6_K step-major: scales and d): mA
         // for the unit's first super-block, mB for its second (SPB == 2) or the next unit's
         // (SPB == 4), one unit half ahead
@@ -665,7 +683,15 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
         // its weights), so the loads in flight at the loop head are counted alike on entry and
         // on the back edge (else the compiler waits for all of them there)
         fm(b_beg, mA);
-        if constexpr (!ORD) {
+        if constexpr (UW) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) fw(s_beg + u, rw[u]);
+            __builtin_amdgcn_sched_barrier(0);
+            load_b(s_beg, std::integral_constant<int, 0>{});
+            load_b(s_beg + 1, std::integral_constant<int, 1>{});
+            load_b(s_beg + 2, std::integral_constant<int, 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+        } else if constexpr (!ORD) {
             load_b(s_beg, std::integral_constant<int, 0>{});
             if constexpr (D >= 3) {
                 load_b(s_beg + 1, std::integral_constant<int, 1>{});
@@ -709,13 +735,23 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
                 // the loads that surely follow step s's activation loads: each step issues its
                 // activation loads, then (after a scheduling fence) at least NW weight loads,
                 // so the weights issued with them and those of steps s + 1 .. s + D - 1
-                sync_loads(std::integral_constant<int, ORD ? NW + (D - 1) * (NDMA + NW) : (D - 1) * NDMA>{});
+                // (UW: the next unit's weights follow the activation loads of its step 0)
+                sync_loads(std::integral_constant<int, UW ? (D - 1) * NDMA + (u >= 1 ? 4 * NW : 0)
+                                                          : ORD ? NW + (D - 1) * (NDMA + NW) : (D - 1) * NDMA>{});
                 // MXFP4: keep each step's decode in its step (hoisted into an earlier one, it
                 // would wait there for weight loads just issued)
                 if constexpr (MX) __builtin_amdgcn_sched_barrier(0);
                 load_b(s + D, std::integral_constant<int, (u + D) & 3>{});
-                if constexpr (ORD) __builtin_amdgcn_sched_barrier(0);
-                fw(s + 3, rw[(u + 3) & 3]);
+                if constexpr (ORD || UW) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (UW) {
+                    if constexpr (u == 0) {
+#pragma unroll
+                        for (int k = 0; k < 4; k++) fw(s0 + 4 + k, rn[k]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                } else {
+                    fw(s + 3, rw[(u + 3) & 3]);
+                }
                 if constexpr (u == 0) fm(b0 + 1, mB);
                 if constexpr (SPB == 2 && u == 2) fm(b0 + 2, mA);
                 mfmas(np_c, nb_c, std::integral_constant<int, u % SPB>{}, u_c, rw[u], (SPB == 2 && u >= 2) ? mB : mA);
@@ -740,12 +776,19 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
                 }
             }
         };
+        auto next = [&]() __attribute__((always_inline)) {
+            if constexpr (UW)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int rb = 0; rb < RB; rb++) rw[k][rb] = rn[k][rb];
+        };
         if constexpr (MX) {
             int s0 = s_beg;
-            for (; s0 + 3 <= s_last; s0 += 4) unit(s0, std::true_type{});
+            for (; s0 + 3 <= s_last; s0 += 4) { unit(s0, std::true_type{}); next(); }
             if (s0 <= s_last) unit(s0, std::false_type{});
         } else {
-            for (int s0 = s_beg; s0 <= s_last; s0 += 4) unit(s0, std::true_type{});
+            for (int s0 = s_beg; s0 <= s_last; s0 += 4) { unit(s0, std::true_type{}); next(); }
         }
         // no load may still be writing the buffers when the workgroup's LDS is released
         __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -853,7 +896,10 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (8 / q16_wpg<SEM, 
                 if constexpr (MX) x0 *= ws;
                 if constexpr (DUAL) {
                     // moe_forward_omp SiLU (QK:2157-2164): clamp to +-80, then silu(g) * u
-                    if (a.clamp_silu) x0 = fminf(fmaxf(x0, -80.0f), 80.0f);
+                    if (a.clamp_silu) {   // (comparisons, as the reference's: a NaN stays)
+                        x0 = x0 < -80.0f ? -80.0f : x0;
+                        x0 = x0 > 80.0f ? 80.0f : x0;
+                    }
                     float x1 = acc[DUAL ? 1 : 0][e][4 * g + r] * is;
                     if constexpr (MX) x1 *= ws;
                     x0 = silu16(x0) * x1;
@@ -1438,6 +1484,12 @@ hipError_t mllm_launch_act16_pro(int sem, const float *x, int ldx, const act16_p
     return hipGetLastError();
 }
 
+// (gate and up in Q6_K run without the step-major metadata)
+bool mllm_q16_tile32(int sem, bool dual)
+{
+    return mllm_q16_mx(sem) || (mllm_q16_supported(sem) && !(dual && (sem == SEM_Q6_K_SEQ || sem == SEM_Q6_K_LOWNIB)));
+}
+
 // Dense launches take 128-entry tiles once there are 256 entries, else 64;
 // grouped launches the bucketing's 64-entry tiles.
 int mllm_q16_tile_entries(bool grouped, int n_entries) { return !grouped && n_entries >= 256 ? 128 : 64; }
@@ -1475,8 +1527,11 @@ hipError_t mllm_launch_q16(int sem, bool dual, const q16_args &a, int max_tiles,
 #define Q16(S)                                                                                   \
     if (sem == S) {                                                                              \
         constexpr bool q6 = S == SEM_Q6_K_SEQ || S == SEM_Q6_K_LOWNIB;                           \
-        if (grouped && a.sm && !dual) return launch16<S, false, 2, true>(a, max_tiles, st);      \
-        if constexpr (!q6) if (grouped && a.sm) return launch16<S, true, 2, true>(a, max_tiles, st); \
+        if (grouped && a.sm && !dual)                                                            \
+            return a.tile32 ? launch16<S, false, 1, true>(a, max_tiles, st) : launch16<S, false, 2, true>(a, max_tiles, st); \
+        if constexpr (!q6) if (grouped && a.sm)                                                  \
+            return a.tile32 ? launch16<S, true, 1, true>(a, max_tiles, st) : launch16<S, true, 2, true>(a, max_tiles, st); \
+        if (grouped && a.tile32) return hipErrorInvalidValue;                                    \
         if (dual) return launch16<S, true, 2, false>(a, max_tiles, st);                          \
         return tm == 128 ? launch16<S, false, 4, false>(a, max_tiles, st) : launch16<S, false, 2, false>(a, max_tiles, st); \
     }
@@ -1486,7 +1541,11 @@ hipError_t mllm_launch_q16(int sem, bool dual, const q16_args &a, int max_tiles,
     Q16(SEM_Q6_K_LOWNIB)
 #undef Q16
     // MXFP4: the grouped expert GEMMs (gate + up fused against fp32 x, down against Q8_0 h)
-    if (sem == SEM_MXFP4 && dual && grouped && a.sm) return launch16<SEM_MXFP4, true, 2, true>(a, max_tiles, st);
-    if (sem == SEM_MXFP4_Q8 && !dual && grouped && a.sm) return launch16<SEM_MXFP4_Q8, false, 2, true>(a, max_tiles, st);
+    if (sem == SEM_MXFP4 && dual && grouped && a.sm)
+        return a.tile32 ? launch16<SEM_MXFP4, true, 1, true>(a, max_tiles, st)
+                        : launch16<SEM_MXFP4, true, 2, true>(a, max_tiles, st);
+    if (sem == SEM_MXFP4_Q8 && !dual && grouped && a.sm)
+        return a.tile32 ? launch16<SEM_MXFP4_Q8, false, 1, true>(a, max_tiles, st)
+                        : launch16<SEM_MXFP4_Q8, false, 2, true>(a, max_tiles, st);
     return hipErrorInvalidValue;
 }

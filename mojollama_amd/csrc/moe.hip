@@ -7,16 +7,17 @@
 // down per type (MXFP4 through Q8_0(h)), combined[n] = sum_k w_k * down_k in
 // k order.
 //
-// Batched flow (T > kMoeDecodeMaxT = 24 tokens):
+// Batched flow (T > 24 tokens, on the fp16-plane GEMM from fewer: moe_grouped):
 //   route -> stable bucketing of the T*K (token, slot) entries by expert on
 //   the GPU -> grouped MFMA GEMM gate+up with the SiLU product in its
 //   epilogue (bucket order) -> grouped MFMA GEMM down -> per-token combine
 //   in k order through the inverse permutation.
-// Decode flow (T <= 24): the same stages with the decode GEMV kernels, one job
+// Decode flow (fewer): the same stages with the decode GEMV kernels, one job
 // per (token, slot), no bucketing.
 #include <stdio.h>
 #include <string.h>
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <vector>
 #include "gemm.h"
@@ -31,7 +32,8 @@ constexpr int kTileEntries = 64;   // entries per grouped-GEMM work tile (gemm.h
 
 // Stable bucketing of entries i = t*K + k by expert idx[i]: entry i lands at
 // pos = off[e] + #{j < i : idx[j] == e}, so each bucket keeps index order
-// (no atomics decide an order).  Two launches over blocks of 1024 entries:
+// (no atomics decide an order).  Two launches over blocks of 1024 entries
+// (one launch where a single block holds them):
 //   k_bucket_rank: per block, an entry's rank among the block's entries of
 //     its expert (its rank among its wave's equal lanes below it -- a 64-step
 //     scan of the wave -- plus that expert's count in the block's earlier
@@ -40,20 +42,20 @@ constexpr int kTileEntries = 64;   // entries per grouped-GEMM work tile (gemm.h
 //     scan over experts of the histogram totals) plus the earlier blocks'
 //     counts give each entry its position: perm[pos] = i, pos_of[i] = pos
 //     (-1 for an expert id outside [0, E)), tok[pos] = i / K when tok is
-//     given; block 0 also writes off[] and the work-tile list (<=
-//     kTileEntries consecutive positions of one expert).
+//     given; block 0 also writes off[] and the work-tile list (<= te
+//     consecutive positions of one expert).
 constexpr int kBucketThreads = 1024, kBucketWaves = kBucketThreads / 64;
 
-__global__ __launch_bounds__(1024) void k_bucket_rank(const int *__restrict__ idx, int TK, int E,
-                                                      int *__restrict__ hist, int *__restrict__ rank)
+// Entry blockIdx.x * 1024 + tid's rank among the block's entries of its expert (e: -1 for an
+// id outside [0, E)), and in thread tid < E the block's count of expert tid.
+__device__ __forceinline__ int bucket_rank(const int *__restrict__ idx, int TK, int E, int &e, int &count)
 {
     __shared__ int wcnt[kBucketWaves][256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int q = tid; q < kBucketWaves * 256; q += kBucketThreads) (&wcnt[0][0])[q] = 0;
     const int i = blockIdx.x * kBucketThreads + tid;
-    int e = i < TK ? idx[i] : -1;
-    const bool valid = e >= 0 && e < E;
-    if (!valid) e = -1;
+    e = i < TK ? idx[i] : -1;
+    if (e < 0 || e >= E) e = -1;
     int r = 0, tot = 0;
     for (int j = 0; j < 64; j++) {
         const int ej = __builtin_amdgcn_readlane(e, j);
@@ -62,38 +64,47 @@ __global__ __launch_bounds__(1024) void k_bucket_rank(const int *__restrict__ id
         r += m & (j < lane);
     }
     __syncthreads();
-    if (valid && r == 0) wcnt[wave][e] = tot;
+    if (e >= 0 && r == 0) wcnt[wave][e] = tot;
     __syncthreads();
-    if (valid) {
+    if (e >= 0)
         for (int w = 0; w < wave; w++) r += wcnt[w][e];
-        rank[i] = r;
-    }
-    if (tid < E) {
-        int h = 0;
-        for (int w = 0; w < kBucketWaves; w++) h += wcnt[w][tid];
-        hist[(long)blockIdx.x * E + tid] = h;
-    }
+    count = 0;
+    if (tid < E)
+        for (int w = 0; w < kBucketWaves; w++) count += wcnt[w][tid];
+    return r;
 }
 
+__global__ __launch_bounds__(1024) void k_bucket_rank(const int *__restrict__ idx, int TK, int E,
+                                                      int *__restrict__ hist, int *__restrict__ rank)
+{
+    int e, count;
+    const int r = bucket_rank(idx, TK, E, e, count);
+    if (e >= 0) rank[blockIdx.x * kBucketThreads + threadIdx.x] = r;
+    if ((int)threadIdx.x < E) hist[(long)blockIdx.x * E + threadIdx.x] = count;
+}
+
+// ONE: a single block, which ranks its entries itself (one launch instead of two of 4.8 us).
+template <bool ONE>
 __global__ __launch_bounds__(1024) void k_bucket_place(const int *__restrict__ idx, int TK, int E, int K, int nblk,
                                                        const int *__restrict__ hist, const int *__restrict__ rank,
                                                        int *__restrict__ off, int *__restrict__ perm,
                                                        int *__restrict__ pos_of, int *__restrict__ tok,
                                                        int *__restrict__ tile_expert, int *__restrict__ tile_begin,
-                                                       int *__restrict__ tile_end, int *__restrict__ n_tiles)
+                                                       int *__restrict__ tile_end, int *__restrict__ n_tiles, int te)
 {
     __shared__ int base[256], scan[256], tbase[256];
     const int tid = threadIdx.x;
     // per expert: its total, and the entries of it in earlier blocks
-    int c = 0, before = 0, nt = 0;
+    int c = 0, before = 0, nt = 0, own = 0, own_e;
+    if constexpr (ONE) own = bucket_rank(idx, TK, E, own_e, c);
     if (tid < 256) {
-        if (tid < E)
+        if (!ONE && tid < E)
             for (int b = 0; b < nblk; b++) {
                 const int h = hist[(long)b * E + tid];
                 c += h;
                 before += b < (int)blockIdx.x ? h : 0;
             }
-        nt = (c + kTileEntries - 1) / kTileEntries;
+        nt = (c + te - 1) / te;
         scan[tid] = c;
         tbase[tid] = nt;
     }
@@ -114,8 +125,8 @@ __global__ __launch_bounds__(1024) void k_bucket_place(const int *__restrict__ i
             const int tb = tbase[tid] - nt;
             for (int t = 0; t < nt; t++) {
                 tile_expert[tb + t] = tid;
-                tile_begin[tb + t] = b + t * kTileEntries;
-                tile_end[tb + t] = b + min(c, (t + 1) * kTileEntries);
+                tile_begin[tb + t] = b + t * te;
+                tile_end[tb + t] = b + min(c, (t + 1) * te);
             }
         }
     }
@@ -128,7 +139,7 @@ __global__ __launch_bounds__(1024) void k_bucket_place(const int *__restrict__ i
     if (i >= TK) return;
     const int e = idx[i];
     if (e >= 0 && e < E) {
-        const int pos = base[e] + rank[i];
+        const int pos = base[e] + (ONE ? own : rank[i]);
         perm[pos] = i;
         pos_of[i] = pos;
         if (tok) tok[pos] = i / K;
@@ -137,15 +148,20 @@ __global__ __launch_bounds__(1024) void k_bucket_place(const int *__restrict__ i
     }
 }
 
-// Both bucketing launches; hist needs (TK/1024 + 1) * E ints and rank TK ints of scratch.
+// The bucketing's launches; hist needs (TK/1024 + 1) * E ints and rank TK ints of scratch.
 hipError_t launch_bucket(const int *idx, int TK, int E, int K, int *hist, int *rank, int *off, int *perm,
                          int *pos_of, int *tok, int *tile_expert, int *tile_begin, int *tile_end, int *n_tiles,
-                         hipStream_t st)
+                         hipStream_t st, int te = kTileEntries)
 {
     const int nblk = (TK + kBucketThreads - 1) / kBucketThreads;
+    if (nblk == 1) {
+        hipLaunchKernelGGL(k_bucket_place<true>, dim3(1), dim3(kBucketThreads), 0, st, idx, TK, E, K, 1, hist, rank,
+                           off, perm, pos_of, tok, tile_expert, tile_begin, tile_end, n_tiles, te);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_bucket_rank, dim3(nblk), dim3(kBucketThreads), 0, st, idx, TK, E, hist, rank);
-    hipLaunchKernelGGL(k_bucket_place, dim3(nblk), dim3(kBucketThreads), 0, st, idx, TK, E, K, nblk, hist, rank,
-                       off, perm, pos_of, tok, tile_expert, tile_begin, tile_end, n_tiles);
+    hipLaunchKernelGGL(k_bucket_place<false>, dim3(nblk), dim3(kBucketThreads), 0, st, idx, TK, E, K, nblk, hist, rank,
+                       off, perm, pos_of, tok, tile_expert, tile_begin, tile_end, n_tiles, te);
     return hipGetLastError();
 }
 
@@ -320,12 +336,45 @@ static int moe_q16_setup(mllm_moe_layer *L)
     return 0;
 }
 
-// Tokens up to which the layer runs the decode GEMVs (one job per (token,
+// Tokens up to which other layers run the decode GEMVs (one job per (token,
 // slot); an expert picked by several tokens is streamed once per token) rather
 // than the bucketed grouped GEMMs.  Measured on MI355X: GPT-OSS shape 225 vs
 // 388 us at T = 16, 407 vs 385 us at T = 32; Qwen3 shape 119 vs 256 us at
 // T = 16, 219 vs 312 us at T = 32, 358 vs 342 us at T = 64.
 constexpr int kMoeDecodeMaxT = 24;
+
+// Layers whose gate/up and down both run on the fp16-plane GEMM with 32-entry tiles.
+static bool moe_q16_small(const mllm_moe_layer &L)
+{
+    return moe_q16_gu(L) && moe_q16_d(L) && L.sm_g && L.sm_d && mllm_q16_tile32(L.sem_g, true) &&
+           mllm_q16_tile32(L.sem_d, false);
+}
+
+// 32-entry tiles while the experts hold few entries on average: twice the workgroups per CU
+// (the launch then streams weights), until experts past 32 entries are decoded twice.
+// Measured, 64- / 32-entry tiles: GPT-OSS T = 16 195 / 182 us, 128 221 / 213, 192 (24 entries
+// an expert) 241 / 220, 256 (32) 258 / 298; Qwen3 T = 64 177 / 162, 256 (16) 185 / 178, 512
+// (32) 212 / 227.  Their list lies in the place of u (moe_forward_impl): TK * M floats.
+static bool moe_tile32(const mllm_moe_layer &L, int T)
+{
+    const long TK = (long)T * L.K;
+    return moe_q16_small(L) && TK <= 24L * L.E && TK * L.M >= 3 * (TK / 32 + L.E + 1) + 1;
+}
+
+// Whether T tokens run the bucketed grouped GEMMs.  Layers on 32-entry tiles take them from
+// the T where streaming each picked expert once (expected number E (1 - (1 - K/E)^T)) costs
+// less than streaming it per token: GEMVs 18 us + bytes at 4.5 TB/s, grouped 45 us + bytes at
+// 2.9 TB/s, fitted to, GEMV / grouped: GPT-OSS T = 8 117 / 127 us, 12 166 / 140, 16 211 / 177,
+// 24 290 / 185; Qwen3 T = 16 103 / 115, 24 135 / 144, 32 175 / 153.
+static bool moe_grouped(const mllm_moe_layer &L, int T)
+{
+    if (T > kMoeDecodeMaxT) return true;
+    if (T <= 8 || !moe_tile32(L, T)) return false;
+    const double mb = 1e-6 * (2.0 * mllm_packed_bytes(mllm_sem_layout(L.sem_g), L.M, L.N, nullptr) +
+                              (double)mllm_packed_bytes(mllm_sem_layout(L.sem_d), L.N, L.M, nullptr));
+    const double picked = L.E * (1.0 - std::pow(1.0 - (double)L.K / L.E, T));
+    return 45.0 + picked * mb / 2.9 < 18.0 + (double)T * L.K * mb / 4.5;
+}
 
 static size_t moe_ws_layout(const mllm_moe_layer &L, int T, moe_ws *w, uint8_t *base)
 {
@@ -506,16 +555,24 @@ static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, floa
 
     // the grouped GEMMs need at least one quant block per row (else the decode
     // GEMVs write the reference's zeros)
-    const bool batched = !L->gemv_only && T > kMoeDecodeMaxT && mllm_qgemm_supported(L->sem_g) && mllm_qgemm_supported(L->sem_u) &&
+    const bool batched = !L->gemv_only && moe_grouped(*L, T) && mllm_qgemm_supported(L->sem_g) && mllm_qgemm_supported(L->sem_u) &&
                          (L->sem_d < 0 || mllm_qgemm_supported(L->sem_d)) &&
                          N >= mllm_sem_block_elems(L->sem_g) && N >= mllm_sem_block_elems(L->sem_u) &&
                          (L->sem_d < 0 || M >= mllm_sem_block_elems(L->sem_d));
     if (batched) {
         if (mllm_sem_uses_q8(L->sem_g) || mllm_sem_uses_q8(L->sem_u))
             CK(mllm_launch_quantize_q8_0(x, T, N, nullptr, q, d, s4, sq, st));
+        const bool t32 = moe_tile32(*L, T);
+        const int te = t32 ? 32 : kTileEntries, max_tiles = TK / te + E + 1;
+        if (t32) {
+            // three lists of max_tiles ints and the count in u's place, which the fp16-plane GEMM leaves free
+            s.tile_expert = (int *)s.u;
+            s.tile_begin = s.tile_expert + max_tiles;
+            s.tile_end = s.tile_begin + max_tiles;
+            s.n_tiles = s.tile_end + max_tiles;
+        }
         CK(launch_bucket(s.idx, TK, E, K, s.bscr, s.bscr + (TK / kBucketThreads + 1) * E, s.off, s.perm, s.pos_of,
-                         s.tok, s.tile_expert, s.tile_begin, s.tile_end, s.n_tiles, st));
-        const int max_tiles = TK / kTileEntries + E + 1;
+                         s.tok, s.tile_expert, s.tile_begin, s.tile_end, s.n_tiles, st, te));
         static_assert(kTileEntries == 64, "the bucketing's tiles are the grouped GEMMs' 64-entry tiles");
         if (moe_q16_gu(*L)) {
             // gate + up + SiLU in bucket order on the fp16-plane GEMM
@@ -529,6 +586,7 @@ static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, floa
             a.out = s.h; a.ldo = M;
             a.n_rows = M; a.n_cols = N; a.n_entries = TK;
             a.tile_expert = s.tile_expert; a.tile_begin = s.tile_begin; a.tile_end = s.tile_end; a.n_tiles = s.n_tiles;
+            a.tile32 = t32;
             a.clamp_silu = L->clamp;
             a.ksplit = 1;
             a.eoff = L->eoff_gu; a.wscale = L->ws_gu;
@@ -573,6 +631,7 @@ static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, floa
             b.out = s.dn; b.ldo = N;
             b.n_rows = N; b.n_cols = M; b.n_entries = TK;
             b.tile_expert = s.tile_expert; b.tile_begin = s.tile_begin; b.tile_end = s.tile_end; b.n_tiles = s.n_tiles;
+            b.tile32 = t32;
             b.ksplit = 1;
             b.eoff = L->eoff_d; b.wscale = L->ws_d;
             CK(mllm_launch_q16(L->sem_d, false, b, max_tiles, st));

@@ -563,3 +563,36 @@ def test_moe_forward_omp_empty_slots(lib, orc):
                         fp(x), n_ff, n_embd, 12, 12, 14, ti.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), fp(tw), 0,
                         fp(out), fp(np.zeros(16, np.float32)), up(np.zeros(64, np.uint8)))
     assert np.all(out == 0.0)
+
+
+@pytest.mark.parametrize("qts,N,M,E,Kk,T", [
+    ((39, 39, 39), 1024, 1024, 8, 4, 20), ((39, 39, 39), 960, 1088, 8, 4, 24), ((12, 12, 14), 1024, 1024, 8, 4, 24),
+    ((39, 39, 39), 192, 320, 20, 3, 100), ((12, 12, 14), 512, 256, 8, 2, 96), ((12, 12, 14), 256, 512, 16, 1, 40),
+    ((39, 39, 39), 64, 64, 256, 1, 25), ((39, 39, 39), 128, 128, 30, 4, 400)])
+def test_moe_layer_32_entry_tiles(dev, orc, qts, N, M, E, Kk, T):
+    """Few entries per expert: the grouped GEMMs on 32-entry tiles, from 9
+    tokens where streaming each picked expert once is cheaper (the first three),
+    with experts of more than 32 entries (one to three tiles) and of none, ragged
+    last rows of a 128-row tile, step counts that are no multiple of four, and
+    the bucketing by one block and by two (1600 entries)."""
+    got, ref = _moe_case(dev, orc, qts, N=N, M=M, E=E, Kk=Kk, T=T, renorm=T % 2, seed=T + N + M)
+    assert O.norm_err(got, ref) < moe_tol(qts)
+
+
+@pytest.mark.parametrize("qts", [(39, 39, 39), (12, 12, 14)])
+def test_moe_layer_32_entry_tiles_nonfinite_token(dev, orc, qts):
+    """A token with an infinite element is routed to no expert (zeros); the others are untouched."""
+    import torch
+    rng = np.random.default_rng(81)
+    N, M, E, Kk, T = 1024, 1024, 8, 4, 24
+    mats = [[W.gen_weights(rng, q, r, c) for _ in range(E)] for q, r, c in zip(qts, (M, M, N), (N, N, M))]
+    router, x = W.gen_router(rng, E, N), W.gen_x(rng, T, N)
+    x[3, 17] = np.inf
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    layer = dev.moe_prepare(qts, N, M, E, Kk, *[[cu(a) for a in m] for m in mats], cu(router), 1)
+    got = layer.forward(cu(x)).cpu().numpy()
+    ri, rw = orc.route(router, x, Kk, 1)
+    ref = np.stack([orc.moe_forward_token(*mats, x[t], M, N, qts, ri[t], rw[t]) if ri[t, 0] >= 0 else np.zeros(N, np.float32)
+                    for t in range(T)])
+    assert ri[3, 0] == -1 and np.all(got[3] == 0.0)
+    assert O.norm_err(got, ref) < moe_tol(qts)
