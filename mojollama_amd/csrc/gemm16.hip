@@ -325,7 +325,7 @@ template <class T> MLLM_DEV T gldo(const void *base, uint32_t off) { return gld<
 // four per CU where 64-entry tiles have two.
 template <int SEM, bool DUAL, int EB> constexpr int q16_waves()   // per SIMD
 {
-    return EB == 1 ? (DUAL ? 3 : 4) : 8 / q16_wpg<SEM, DUAL, EB>();
+    return EB == 1 ? (DUAL ? 3 : 4) : q16_traits<SEM>::MX && DUAL ? 3 : 8 / q16_wpg<SEM, DUAL, EB>();
 }
 
 template <int SEM, bool DUAL, int EB, bool SM>
@@ -408,12 +408,16 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (q16_waves<SEM, DU
     // MFMA reads of 16 lanes (rows r .. r+15, one chunk each) fall in distinct banks.
     // Buffers, each its own LDS object: the compiler then tracks which outstanding loads
     // write which buffer.  One plane: buffer = step % 4, loads run three steps ahead; two
-    // planes, MXFP4: buffer = 2 (step % 4) + plane, three steps ahead (eight buffers); two
-    // planes, K-quants: buffer = 2 (step % 2) + plane, one step ahead.
+    // planes with eight buffers: buffer = 2 (step % 4) + plane, three steps ahead; two
+    // planes with four: buffer = 2 (step % 2) + plane, one step ahead.
     // load instructions per wave, plane and step (four waves: EB; MXFP4's eight: one, for
     // waves whose rows the tile's entry blocks reach)
     constexpr int NCH = TM * 8 / (64 * WPG);
-    constexpr bool B8 = MX || EB == 1;   // larger K-quant tiles keep four buffers (their LDS then admits a third workgroup per CU)
+    // larger K-quant tiles and MXFP4's fused gate + up keep four buffers: their LDS (and
+    // registers) then admit a third workgroup per CU (GPT-OSS T = 1280: 2 workgroups with
+    // loads three steps ahead 631.7 us, 3 with one step ahead 618.5; the eight-wave MXFP4
+    // down measured no gain, 616.2 -> 620.5)
+    constexpr bool B8 = (MX && !DUAL) || EB == 1;
     constexpr int D2 = B8 ? 3 : 1;      // two-plane prefetch distance (steps)
     constexpr bool UW = MX && EB == 1 && !DUAL;   // weights fetched a unit (four steps) at a time, see main_loop
     __shared__ __attribute__((aligned(16))) _Float16 sB0[TM * 64], sB1[TM * 64], sB2[TM * 64], sB3[TM * 64];
@@ -896,17 +900,15 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (q16_waves<SEM, DU
                 if constexpr (MX) x0 *= ws;
                 if constexpr (DUAL) {
                     // moe_forward_omp SiLU (QK:2157-2164): clamp to +-80, then silu(g) * u
-                    if (a.clamp_silu) {   // (comparisons, as the reference's: a NaN stays)
-                        x0 = x0 < -80.0f ? -80.0f : x0;
-                        x0 = x0 > 80.0f ? 80.0f : x0;
-                    }
+                    // (the reference's comparisons keep a NaN)
+                    if (a.clamp_silu) x0 = x0 == x0 ? __builtin_amdgcn_fmed3f(x0, -80.0f, 80.0f) : x0;
                     float x1 = acc[DUAL ? 1 : 0][e][4 * g + r] * is;
                     if constexpr (MX) x1 *= ws;
                     x0 = silu16(x0) * x1;
                 }
                 v[r] = x0;
             }
-            if (a.add && a.ksplit <= 1) {   // the residual, read by the lane that writes its place
+            if constexpr (!DUAL && !SM) if (a.add && a.ksplit <= 1) {   // the residual, read by the lane that writes its place
                 const float *ad = a.add + orow * ldo + n;
 #pragma unroll
                 for (int r = 0; r < 4; r++)
