@@ -308,7 +308,8 @@ MLLM_API int mllm_dequant(int sem, const void *packed_dev, int n_rows, int n_col
  * (CE:606-638), renormalised when `renorm` (GO:88-92): gate/up per type,
  * SiLU with the gate clamped to +-80, down per type, k-order combine.
  * T > 24 tokens run the batched path (GPU bucketing by expert, grouped MFMA
- * GEMMs); T <= 24 the decode GEMVs, one job per (token, slot). */
+ * GEMMs), MXFP4 and Q4_K / Q6_K layers from 9 tokens where their size makes it
+ * faster; fewer the decode GEMVs, one job per (token, slot). */
 typedef struct mllm_moe_layer mllm_moe_layer;
 MLLM_API mllm_moe_layer *mllm_moe_prepare(int qt_gate, int qt_up, int qt_down, int N, int M, int E, int K,
                                           const void *const *gate_packed, const void *const *up_packed,
@@ -377,7 +378,7 @@ typedef struct {
  * seq_lens[b] cached rows (device array, each <= max_seq).
  * mode 0: CE:141-158 gqa (expf weights, 1 / sum); mode 1: gqa_attention.c
  * (see gqa_attention_decode).  q, out [B][NH * HD]; NH % NKH == 0,
- * NH / NKH <= 16, HD <= 256 and a multiple of 4; K and V 16-byte aligned.  Three launches on `stream`; weights and partial
+ * NH / NKH <= 16, HD <= 256 and a multiple of 4; K and V 16-byte aligned.  Two or three launches on `stream`; scores and partial
  * sums go to the workspace (mllm_gqa_workspace_size). */
 MLLM_API long mllm_gqa_workspace_size(int B, int NH, int HD, int max_seq);
 MLLM_API int mllm_gqa_decode(int mode, const float *q, const mllm_kv_view *kv, const int *seq_lens, int max_seq, int B,
@@ -414,7 +415,7 @@ MLLM_API mllm_gptoss *mllm_gptoss_create(const mllm_gptoss_desc *desc);
 MLLM_API void mllm_gptoss_release(mllm_gptoss *m);
 /* Floats of one of the step's K / V caches: L * max_ctx * NKH * HD. */
 MLLM_API long mllm_gptoss_kv_floats(const mllm_gptoss *m);
-/* One token, device pointers only, no host synchronisation (14 launches per
+/* One token, device pointers only, no host synchronisation (12 launches per
  * layer; capturable): x_emb the token's embedding row [N], pos the RoPE
  * position [1], kv_len [L] (read, then incremented), caches [L][max_ctx][NKH *
  * HD], logits [outNR]. */

@@ -459,6 +459,36 @@ __global__ void k_rope(float *buf, int NH, int HD, const int *pos, const float *
     }
 }
 
+// mllm_rope_append: grid (NH + 2 NKH) heads, one wave each.  One launch of a decode step's
+// layer instead of two (4.1 and 2.3 us, latency).
+__global__ __launch_bounds__(64) void k_rope_append(float *qkv, int NH, int NKH, int HD, const int *pos,
+                                                    const float *cos_t, const float *sin_t, int r, mllm_kv_view kv,
+                                                    const int *kv_pos)
+{
+    const int h = blockIdx.x, hd2 = r / 2;
+    const float *src = qkv + (long)h * HD;
+    float *dst = qkv + (long)h * HD;
+    if (h >= NH) {
+        const int j = (h - NH) % NKH, s = kv_pos[0];
+        const float *row = s < 0 ? nullptr : kv_row(kv.k, kv, 0, s, NKH, HD, j);
+        if (!row) return;
+        dst = (h < NH + NKH ? kv.k : kv.v) + (row - kv.k);
+    }
+    if (h >= NH + NKH) {
+        for (int i = threadIdx.x; i < HD; i += 64) dst[i] = src[i];
+        return;
+    }
+    const long p = pos[0];
+    for (int i = threadIdx.x; i < hd2; i += 64) {
+        const float a0 = src[i], a1 = src[i + hd2];
+        const float cs = cos_t[p * hd2 + i], sn = sin_t[p * hd2 + i];
+        dst[i] = a0 * cs - a1 * sn;
+        dst[i + hd2] = a1 * cs + a0 * sn;
+    }
+    if (h >= NH)
+        for (int i = r + threadIdx.x; i < HD; i += 64) dst[i] = src[i];
+}
+
 long a256(long n) { return (n + 255) / 256 * 256; }
 
 // Workspace carve-up of mllm_gqa_decode.
@@ -579,6 +609,24 @@ MLLM_API int mllm_rope(float *buf, int T, int NH, int HD, const int *pos, const 
     hipLaunchKernelGGL(k_rope, dim3(T), dim3(256), 0, (hipStream_t)stream, buf, NH, HD, pos, cos_t, sin_t, r);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
+
+} // extern "C"
+
+int mllm_rope_append(float *qkv, int NH, int NKH, int HD, const int *pos, const float *cos_t, const float *sin_t,
+                     int rope_dim, const mllm_kv_view *kv, const int *kv_pos, hipStream_t st)
+{
+    const int r = rope_dim <= 0 ? HD : rope_dim;
+    if (!qkv || !pos || !cos_t || !sin_t || !kv || !kv->k || !kv->v || !kv_pos || NH <= 0 || NKH <= 0 || HD <= 0 ||
+        r > HD || (r & 1)) {
+        mllm_set_error("mllm_rope_append: bad arguments");
+        return -1;
+    }
+    hipLaunchKernelGGL(k_rope_append, dim3(NH + 2 * NKH), dim3(64), 0, st, qkv, NH, NKH, HD, pos, cos_t, sin_t, r, *kv,
+                       kv_pos);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+extern "C" {
 
 // ------------------------------------------------------------ page table
 // CE:160-201: a free list initialised so that allocation hands out pages

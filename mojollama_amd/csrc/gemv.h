@@ -188,8 +188,9 @@ hipError_t mllm_launch_silu_mul(const float *g, const float *u, float *h, long n
 // out[t][i] = sum_k (in k order) w[t][k] * d[t][k][i]; fused selects fmaf (moe_ffn CE:662) or
 // add-of-product (moe_forward_omp QK:2243-2244).  d == nullptr: every d term is 0.  Slots whose
 // expert idx[t][k] is negative (left empty by the routing) are skipped; idx == nullptr: none are.
+// base (optional, out's layout, may be out): out = base + that sum.
 hipError_t mllm_launch_combine(const float *d, const float *w, const int *idx, int T, int K, int N, float *out,
-                               int fused, hipStream_t st);
+                               int fused, hipStream_t st, const float *base = nullptr);
 
 // fp32 rows of a packed matrix under a fp32-weight semantic; returns 0 or -1
 // (semantic without an fp32 weight form, or launch failure).

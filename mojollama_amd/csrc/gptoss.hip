@@ -1,19 +1,19 @@
 // gptoss.hip — gptoss_forward (GO:96-189) on the GPU: one decode token
 // through every layer with the weights resident in HBM.
 //
-// Per layer (14 launches, all on one stream, no host synchronisation, so a
+// Per layer (12 launches, all on one stream, no host synchronisation, so a
 // step can be captured in a graph):
 //   qkv  = Wqkv (rms(x) * wAN)        one MXFP4 GEMV over the stacked q/k/v
 //                                     rows with the RMS norm in its prologue
-//   RoPE on the q and k heads          one launch over NH + NKH heads
-//   K/V row kv_len[l] := k, v          mllm_kv_append
+//   RoPE on the q and k heads,         one launch over NH + 2 NKH heads
+//   K/V row kv_len[l] := k, v          (mllm_rope_append)
 //   att  = attention over kv_len[l]+1  mllm_gqa_decode, gqa_attention.c softmax
 //   x2   = x + Wo att                  GEMV with the residual in its epilogue
 //   xn   = rms(x2) * wFN               the prologue kernel on its own (the
 //                                      router and the experts both read it)
-//   ffn  = MoE layer (route + experts) mllm_moe_forward, moe_forward_omp's
-//                                      semantics, GO's renormalised router
-//   x   += ffn                         x is still the layer's input: GO:186
+//   x   += MoE layer (route + experts) mllm_moe_forward_add, moe_forward_omp's
+//                                      semantics, GO's renormalised router;
+//                                      x is still the layer's input: GO:186
 //                                      adds the FFN to res, not to x2
 // then logits = Wout xn (the last layer's xn, GO:189) and kv_len[l] += 1.
 #include <string.h>
@@ -52,7 +52,7 @@ struct mllm_gptoss {
     uint8_t *wout = nullptr;
     float *cos_t = nullptr, *sin_t = nullptr;
     // step buffers
-    float *x = nullptr, *xn = nullptr, *x2 = nullptr, *qkvb = nullptr, *att = nullptr, *ffn = nullptr;
+    float *x = nullptr, *xn = nullptr, *x2 = nullptr, *qkvb = nullptr, *att = nullptr;
     int *len1 = nullptr;
     uint8_t *ws = nullptr;
     long ws_gemv = 0, ws_attn = 0, ws_moe = 0;
@@ -166,7 +166,6 @@ MLLM_API mllm_gptoss *mllm_gptoss_create(const mllm_gptoss_desc *desc)
         m->x = (float *)m->dalloc((size_t)N * 4);
         m->xn = (float *)m->dalloc((size_t)N * 4);
         m->x2 = (float *)m->dalloc((size_t)N * 4);
-        m->ffn = (float *)m->dalloc((size_t)N * 4);
         m->qkvb = (float *)m->dalloc((size_t)(inner + 2 * kvd) * 4);
         m->att = (float *)m->dalloc((size_t)inner * 4);
         m->len1 = (int *)m->dalloc((size_t)d.L * 4);
@@ -184,7 +183,7 @@ MLLM_API mllm_gptoss *mllm_gptoss_create(const mllm_gptoss_desc *desc)
         m->ws_moe = mllm_moe_workspace_size(m->moe[0], 1);
         m->ws_bytes = a256(m->ws_gemv) + a256(m->ws_attn) + a256(m->ws_moe);
         m->ws = (uint8_t *)m->dalloc(m->ws_bytes);
-        ok = m->x && m->xn && m->x2 && m->ffn && m->qkvb && m->att && m->len1 && m->ws && g1 >= 0 && g2 >= 0 &&
+        ok = m->x && m->xn && m->x2 && m->qkvb && m->att && m->len1 && m->ws && g1 >= 0 && g2 >= 0 &&
              g3 >= 0 && m->ws_moe > 0;
     }
     if (!ok) {
@@ -223,17 +222,15 @@ MLLM_API int mllm_gptoss_step(mllm_gptoss *m, const float *x_emb, const int *pos
         fq.rms_eps = d.eps;
         fq.rms_div = 1;
         CKI(mllm_gemv_fused(SEM_MXFP4, m->qkv[l], m->x, m->qkvb, inner + 2 * kvd, N, 1, &fq, ws_g, st));
-        CKI(mllm_rope(m->qkvb, 1, d.NH + d.NKH, d.HD, pos, m->cos_t, m->sin_t, d.rope_dim, st));
         mllm_kv_view kv{k_cache + l * layer, v_cache + l * layer, 0, nullptr, 0, 0, 0};
-        CKI(mllm_kv_append(&kv, kv_len + l, m->qkvb + inner, m->qkvb + inner + kvd, 1, d.NKH, d.HD, st));
+        CKI(mllm_rope_append(m->qkvb, d.NH, d.NKH, d.HD, pos, m->cos_t, m->sin_t, d.rope_dim, &kv, kv_len + l, st));
         CKI(mllm_gqa_decode(1, m->qkvb, &kv, m->len1 + l, d.max_ctx, 1, d.NH, d.NKH, d.HD, m->att, ws_a,
                             m->ws_attn, st));
         mllm_gemv_fusion fo{};
         fo.out_add = m->x;
         CKI(mllm_gemv_fused(SEM_MXFP4, m->wo[l], m->att, m->x2, N, inner, 1, &fo, ws_g, st));
         CK(mllm_launch_act_prologue(m->x2, nullptr, nullptr, m->fn[l], d.eps, 1, nullptr, 1, 1, N, N, m->xn, st));
-        CKI(mllm_moe_forward(m->moe[l], m->xn, 1, m->ffn, ws_m, m->ws_moe, nullptr, nullptr, st));
-        CK(mllm_launch_add(m->x, m->ffn, N, st));
+        CKI(mllm_moe_forward_add(m->moe[l], m->xn, 1, m->x, m->x, ws_m, m->ws_moe, st));
     }
     CKI(mllm_gemv(SEM_MXFP4, m->wout, m->xn, logits, d.outNR, N, 1, ws_g, st));
     hipLaunchKernelGGL(k_len_increment, dim3((d.L + 255) / 256), dim3(256), 0, st, kv_len, d.L);

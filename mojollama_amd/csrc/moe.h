@@ -38,6 +38,16 @@ void mllm_gptoss_cache_clear();
 int mllm_moe_forward_routed(const mllm_moe_layer *L, const float *x, int T, float *out, void *workspace,
                             long ws_bytes, const int *idx, const float *w, hipStream_t st);
 
+// mllm_moe_forward with a residual: out = base + the layer's output (base may be out).
+int mllm_moe_forward_add(const mllm_moe_layer *L, const float *x, int T, const float *base, float *out,
+                         void *workspace, long ws_bytes, hipStream_t st);
+
+// One decode token's RoPE and KV append in one launch (mllm_rope over the q and k heads,
+// mllm_kv_append): qkv [NH + 2 NKH][HD] (k and v after q), q rotated in place, the rotated k
+// and v written to cache row kv_pos[0] of kv's first sequence.
+int mllm_rope_append(float *qkv, int NH, int NKH, int HD, const int *pos, const float *cos_t, const float *sin_t,
+                     int rope_dim, const mllm_kv_view *kv, const int *kv_pos, hipStream_t st);
+
 // A layer for routed forwards over the expert types of moe_forward_omp (GGUF
 // codes, QK:2094-2245) and the device table tab_dev ([E] gate, [E] up, [E]
 // down packed views; the caller's, kept alive while the layer is used).  No

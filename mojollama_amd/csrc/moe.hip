@@ -171,7 +171,7 @@ size_t bucket_scratch_ints(int TK, int E) { return (size_t)(TK / kBucketThreads 
 // moe_forward_omp's combined[row] += top_weight * dot (QK:2243-2244); every dn
 // term is 0 when dn is null (a down type the reference leaves at zero).
 __global__ void k_combine_pos(const float *__restrict__ dn, const float *__restrict__ w,
-                              const int *__restrict__ pos_of, int K, int N, float *__restrict__ out)
+                              const int *__restrict__ pos_of, int K, int N, float *out, const float *base)
 {
     // four consecutive n per thread (N % 4 == 0: 16-byte loads), the same
     // per-element arithmetic as one n per thread
@@ -186,11 +186,15 @@ __global__ void k_combine_pos(const float *__restrict__ dn, const float *__restr
         const float4 v = dn ? *reinterpret_cast<const float4 *>(dn + (long)pos * N + n) : make_float4(0.f, 0.f, 0.f, 0.f);
         acc.x += wk * v.x; acc.y += wk * v.y; acc.z += wk * v.z; acc.w += wk * v.w;
     }
+    if (base) {
+        const float4 b = *reinterpret_cast<const float4 *>(base + (long)t * N + n);
+        acc = make_float4(b.x + acc.x, b.y + acc.y, b.z + acc.z, b.w + acc.w);
+    }
     *reinterpret_cast<float4 *>(out + (long)t * N + n) = acc;
 }
 
 __global__ void k_combine_pos1(const float *__restrict__ dn, const float *__restrict__ w,
-                               const int *__restrict__ pos_of, int K, int N, float *__restrict__ out)
+                               const int *__restrict__ pos_of, int K, int N, float *out, const float *base)
 {
     const int t = blockIdx.y;
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
@@ -200,7 +204,7 @@ __global__ void k_combine_pos1(const float *__restrict__ dn, const float *__rest
         const int pos = pos_of[t * K + k];
         if (pos >= 0) acc += w[t * K + k] * (dn ? dn[(long)pos * N + n] : 0.0f);
     }
-    out[(long)t * N + n] = acc;
+    out[(long)t * N + n] = base ? base[(long)t * N + n] + acc : acc;
 }
 
 size_t a256(size_t n) { return (n + 255) / 256 * 256; }
@@ -529,10 +533,11 @@ MLLM_API int mllm_moe_layer_info(const mllm_moe_layer *L)
 
 // x [T][N] fp32 -> out [T][N].  Routing from the layer's router, or, with
 // idx_in / w_in (device [T][K]), the caller's (moe_forward_omp's own contract,
-// QK:2066-2071).  idx_out / w_out (optional) receive the routing used.
+// QK:2066-2071).  idx_out / w_out (optional) receive the routing used.  base (optional, may be
+// out): out = base + the layer's output.
 static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, float *out, void *workspace,
                             long ws_bytes, int *idx_out, float *w_out, const int *idx_in, const float *w_in,
-                            hipStream_t st)
+                            hipStream_t st, const float *base = nullptr)
 {
     if (!L || T <= 0) return -1;
     if (ws_bytes < (long)moe_ws_layout(*L, T, nullptr, nullptr)) return -1;
@@ -651,12 +656,12 @@ static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, floa
             b.tile_expert = s.tile_expert; b.tile_begin = s.tile_begin; b.tile_end = s.tile_end; b.n_tiles = s.n_tiles;
             CK(mllm_launch_qgemm(L->sem_d, xmode_of(L->sem_d), false, b, max_tiles, st));
         }
-        if (N % 4 == 0 && ((uintptr_t)out & 15) == 0)
+        if (N % 4 == 0 && (((uintptr_t)out | (uintptr_t)base) & 15) == 0)
             hipLaunchKernelGGL(k_combine_pos, dim3((N / 4 + 255) / 256, T), dim3(256), 0, st,
-                               L->sem_d >= 0 ? s.dn : nullptr, s.w, s.pos_of, K, N, out);
+                               L->sem_d >= 0 ? s.dn : nullptr, s.w, s.pos_of, K, N, out, base);
         else
             hipLaunchKernelGGL(k_combine_pos1, dim3((N + 255) / 256, T), dim3(256), 0, st,
-                               L->sem_d >= 0 ? s.dn : nullptr, s.w, s.pos_of, K, N, out);
+                               L->sem_d >= 0 ? s.dn : nullptr, s.w, s.pos_of, K, N, out, base);
         CK(hipGetLastError());
     } else {
         // decode: one GEMV launch per projection over all T*K (token, slot)
@@ -681,7 +686,7 @@ static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, floa
             b.out = s.dn; b.out_job_stride = N; b.ldo = N;
             b.n_rows = N; b.n_cols = M; b.B = 1;
             CK(mllm_launch_gemv(L->sem_d, b, TK, st));
-            CK(mllm_launch_combine(s.dn, s.w, s.idx, T, K, N, out, 0, st));
+            CK(mllm_launch_combine(s.dn, s.w, s.idx, T, K, N, out, 0, st, base));
             if (idx_out) CK(hipMemcpyAsync(idx_out, s.idx, (size_t)TK * 4, hipMemcpyDeviceToDevice, st));
             if (w_out) CK(hipMemcpyAsync(w_out, s.w, (size_t)TK * 4, hipMemcpyDeviceToDevice, st));
             return 0;
@@ -710,7 +715,7 @@ static int moe_forward_impl(const mllm_moe_layer *L, const float *x, int T, floa
             }
             CK(mllm_launch_gemv(L->sem_d, b, TK, st));
         }
-        CK(mllm_launch_combine(L->sem_d >= 0 ? s.dn : nullptr, s.w, s.idx, T, K, N, out, 0, st));
+        CK(mllm_launch_combine(L->sem_d >= 0 ? s.dn : nullptr, s.w, s.idx, T, K, N, out, 0, st, base));
     }
     if (idx_out) CK(hipMemcpyAsync(idx_out, s.idx, (size_t)TK * 4, hipMemcpyDeviceToDevice, st));
     if (w_out) CK(hipMemcpyAsync(w_out, s.w, (size_t)TK * 4, hipMemcpyDeviceToDevice, st));
@@ -723,6 +728,12 @@ int mllm_moe_forward_routed(const mllm_moe_layer *L, const float *x, int T, floa
 {
     if (!idx || !w) return -1;
     return moe_forward_impl(L, x, T, out, workspace, ws_bytes, nullptr, nullptr, idx, w, st);
+}
+
+int mllm_moe_forward_add(const mllm_moe_layer *L, const float *x, int T, const float *base, float *out,
+                         void *workspace, long ws_bytes, hipStream_t st)
+{
+    return moe_forward_impl(L, x, T, out, workspace, ws_bytes, nullptr, nullptr, nullptr, nullptr, st, base);
 }
 
 mllm_moe_layer *mllm_moe_layer_for_codes(int qt_gate, int qt_up, int qt_down, int N, int M, int E, int K,

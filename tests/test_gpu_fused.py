@@ -216,3 +216,25 @@ def test_fused_silu_pair_batched(dev, orc, sem, R, C, B, mode):
     err = O.norm_err(got, ref)
     print(f"[parity] fused pair {K.SEM_NAMES[sem]} {R}x{C} B={B} {mode}: {err:.3e}", flush=True)
     assert err < tol, K.last_error(dev.so)
+
+
+@pytest.mark.parametrize("C,ld,B", [(2880, 2881, 3), (17408, 17408, 9), (67584, 67584, 9), (5120, 5123, 9)])
+def test_fused_prologue_kernel_rows(dev, orc, C, ld, B):
+    """The standalone prologue's forms: rows and strides that are no multiple of
+    four elements (scalar accesses), rows of several groups per thread, and rows
+    longer than its registers hold (scalar past 4096, vector past 16384)."""
+    import torch
+    rng = np.random.default_rng(C + B)
+    R, sem = 40, K.MXFP4
+    w = W.gen_weights(rng, 39, R, C)
+    x, res = W.gen_x(rng, B, ld), W.gen_x(rng, B, ld)
+    g = (rng.standard_normal(C) * 0.5 + 1.0).astype(np.float32)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    packed, xt, rt, gt = dev.pack(sem, cu(w), R, C), cu(x), cu(res), cu(g)
+    res_out = torch.zeros(B, ld, device="cuda")
+    f = dev.fusion(x_res=rt, res_out=res_out, rms_w=gt, rms_eps=1e-5, x_ld=ld)
+    got = dev.gemv_fused(sem, packed, xt.data_ptr(), R, C, f, B=B).cpu().numpy()
+    v = (x + res)[:, :C]
+    assert np.array_equal(res_out.cpu().numpy()[:, :C], v)
+    ref = orc.gemv(sem, w, np.ascontiguousarray(rms_np(v, g, 1e-5, False), np.float32), R, C, B)
+    assert O.norm_err(got, ref) < GEMV_TOL
