@@ -34,9 +34,21 @@ int mf_min_batch(int sem, int n_rows)
 }
 int mf_block(int sem) { return (sem == SEM_Q4_K_GGML || sem == SEM_Q6_K_SEQ) ? 256 : 32; }
 
+// Rows short enough that a workgroup stages all of them in one or two passes and each wave
+// has few units stay whole: a split saves little there, and the launch that joins it costs
+// more.  Four blocks and a head of 1024 rows, B = 8, split / whole: N = 1024 Q4_K 172.7 /
+// 150.4 us, Q8_0 200.6 / 176.3, MXFP4 179.5 / 171.0, Q4_0 175.9 / 143.4; N = 2048 Q4_K 216.9 /
+// 211.0, Q4_0 200.0 / 200.1, but MXFP4 215.5 / 222.3 and Q8_0 234.3 / 240.0; 4096 columns of
+// Q4_K, B = 3, 246.5 / 252.9.  Fewer than 32 tiles (an eighth of the CUs) were not tried.
+constexpr int kMfWholeTiles = 32;
+int mf_whole_cols(int sem)
+{
+    return sem == SEM_Q4_K_GGML || sem == SEM_Q6_K_SEQ || sem == SEM_Q4_0 ? 2304 : 1536;
+}
+
 // S: the fewest K splits whose range fits the LDS budget, raised (up to 8
 // and one 256-element block per split) until rows x splits give a tile per
-// CU; without a partials buffer only S = 1.
+// CU (but see kMfWholeTiles); without a partials buffer only S = 1.
 mf_plan mf_plan_for(int sem, int n_rows, int n_cols, int B, bool pro, bool pair, bool have_part)
 {
     mf_plan p{};
@@ -54,7 +66,8 @@ mf_plan mf_plan_for(int sem, int n_rows, int n_cols, int B, bool pro, bool pair,
     const int smax = std::min(nb, kMfMaxSplits);
     while (S < smax && lds_for(S) > (size_t)kMfLdsCap) S++;
     if (lds_for(S) > (size_t)kMfLdsCap) return p;
-    while (S < smax && (long)p.n_tiles * S < cus) S++;
+    if (S > 1 || p.n_tiles < kMfWholeTiles || n_cols > mf_whole_cols(sem))
+        while (S < smax && (long)p.n_tiles * S < cus) S++;
     if (!have_part) {
         if (lds_for(1) > (size_t)kMfLdsCap) return p;
         S = 1;
