@@ -216,8 +216,11 @@ __global__ __launch_bounds__(256, 4) void k_attn_scores(attn_args a)
         const int n = HD - s * kSeg;   // elements left (a segment's pieces past them are zeros)
         if (!all || n < kSeg) {
 #pragma unroll
-            for (int k = 0; k < 8; k++)
-                if (4 * pc >= n || __shfl(ro, 8 * k + (lane >> 3), 64) < 0) v[0][k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            for (int k = 0; k < 8; k++) {
+                // with every lane active: lanes past the row's end hold offsets that the others read
+                const bool miss = __shfl(ro, 8 * k + (lane >> 3), 64) < 0;
+                if (miss || 4 * pc >= n) v[0][k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
         }
 #pragma unroll
         for (int k = 0; k < 8; k++) *reinterpret_cast<float4 *>(kw + (8 * k + (lane >> 3)) * kSegLd + 4 * pc) = v[0][k];

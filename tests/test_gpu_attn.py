@@ -297,3 +297,33 @@ def test_gqa_decode_edges(dev, orc, mode, nh, nkh, hd, S_list, page):
         ref = orc.gqa_decode(mode, q[b], k[b], v[b], S, nh, nkh, hd)
         err = np.max(np.abs(got[b] - ref))
         assert err <= attn_tol(orc, mode, q[b], k[b], v[b], S, nh, nkh, hd, ref), (b, S, err, np.max(np.abs(ref)))
+
+
+@pytest.mark.parametrize("mode", [O.ATTN_CE, O.ATTN_GQA_C])
+@pytest.mark.parametrize("nh,nkh,hd", [(8, 2, 16), (8, 2, 36), (4, 4, 48), (24, 3, 80), (16, 1, 112), (6, 2, 64), (4, 2, 20)])
+def test_gqa_decode_unmapped_pages_any_head_size(dev, orc, mode, nh, nkh, hd):
+    """Rows on an entry of -1, on one past the pool and past the table's reach read
+    as zeros at head sizes that end inside a 32-element segment; the pool's page 0,
+    which no sequence maps, holds NaN and an infinity."""
+    import torch
+    rng = np.random.default_rng(hd + 7 * mode)
+    ps, S = 16, 150
+    q, k, v = make_case(rng, 2, [S, S], nh, nkh, hd)
+    kp, vp, tables, n_pages = paged_copy(rng, k, v, [S, S], ps, nkh, hd)
+    kp = np.concatenate([np.full_like(kp[:1], np.nan), kp])
+    vp = np.concatenate([np.full_like(vp[:1], np.inf), vp])
+    tables, n_pages = tables + 1, n_pages + 1
+    tables[0, 1], tables[1, 0], tables[1, 5] = -1, n_pages, -7
+    tables = tables[:, :9]                        # positions 144 .. 149 lie past max_blocks
+    k[0, 16:32], v[0, 16:32] = 0, 0
+    for x in (k[1], v[1]):
+        x[0:16], x[80:96] = 0, 0
+    k[:, 144:], v[:, 144:] = 0, 0
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    kv = dev.kv_view(cu(kp), cu(vp), block_tables=cu(tables), page_size=ps, n_pages=n_pages)
+    lens = torch.tensor([S, S], dtype=torch.int32, device="cuda")
+    got = dev.gqa_decode(mode, cu(q), kv, lens, S, nh, nkh, hd).cpu().numpy()
+    for b in range(2):
+        ref = orc.gqa_decode(mode, q[b], k[b], v[b], S, nh, nkh, hd)
+        err = np.max(np.abs(got[b] - ref))
+        assert err <= attn_tol(orc, mode, q[b], k[b], v[b], S, nh, nkh, hd, ref), (b, err, np.max(np.abs(ref)))
