@@ -739,21 +739,24 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (q16_waves<SEM, DU
                 // the loads that surely follow step s's activation loads: each step issues its
                 // activation loads, then (after a scheduling fence) at least NW weight loads,
                 // so the weights issued with them and those of steps s + 1 .. s + D - 1
-                // (UW: the next unit's weights follow the activation loads of its step 0)
-                sync_loads(std::integral_constant<int, UW ? (D - 1) * NDMA + (u >= 1 ? 4 * NW : 0)
-                                                          : ORD ? NW + (D - 1) * (NDMA + NW) : (D - 1) * NDMA>{});
+                // (UW: the next unit's weights follow the activation loads of its step 0).  A short
+                // unit's steps issue no weights (no step is left to read them), so past its first
+                // step only activation loads are counted
+                sync_loads(std::integral_constant<int, !full && u >= 1 ? (D - 1) * NDMA
+                                                       : UW ? (D - 1) * NDMA + (u >= 1 ? 4 * NW : 0)
+                                                       : ORD ? NW + (D - 1) * (NDMA + NW) : (D - 1) * NDMA>{});
                 // MXFP4: keep each step's decode in its step (hoisted into an earlier one, it
                 // would wait there for weight loads just issued)
                 if constexpr (MX) __builtin_amdgcn_sched_barrier(0);
                 load_b(s + D, std::integral_constant<int, (u + D) & 3>{});
                 if constexpr (ORD || UW) __builtin_amdgcn_sched_barrier(0);
                 if constexpr (UW) {
-                    if constexpr (u == 0) {
+                    if constexpr (full && u == 0) {
 #pragma unroll
                         for (int k = 0; k < 4; k++) fw(s0 + 4 + k, rn[k]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                } else {
+                } else if constexpr (full) {
                     fw(s + 3, rw[(u + 3) & 3]);
                 }
                 if constexpr (u == 0) fm(b0 + 1, mB);
@@ -765,7 +768,7 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (q16_waves<SEM, DU
             if constexpr (MX) {
                 if (full || s0 + 1 <= s_last) one(std::integral_constant<int, 1>{});
                 if (full || s0 + 2 <= s_last) one(std::integral_constant<int, 2>{});
-                if (full || s0 + 3 <= s_last) one(std::integral_constant<int, 3>{});
+                if constexpr (full) one(std::integral_constant<int, 3>{});
             } else if constexpr (SPB == 4) {
                 one(std::integral_constant<int, 1>{});
                 one(std::integral_constant<int, 2>{});

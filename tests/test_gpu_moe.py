@@ -596,3 +596,28 @@ def test_moe_layer_32_entry_tiles_nonfinite_token(dev, orc, qts):
                     for t in range(T)])
     assert ri[3, 0] == -1 and np.all(got[3] == 0.0)
     assert O.norm_err(got, ref) < moe_tol(qts)
+
+
+@pytest.mark.parametrize("N,M,E,Kk,T", [(128, 192, 16, 4, 30), (192, 128, 16, 4, 30), (640, 704, 16, 4, 40),
+                                        (704, 640, 16, 4, 40), (640, 704, 64, 4, 300), (128, 192, 4, 2, 100),
+                                        (640, 704, 4, 2, 60), (704, 640, 4, 2, 200), (896, 192, 4, 2, 140)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_moe_layer_mxfp4_short_last_unit(dev, orc, N, M, E, Kk, T, bf16):
+    """MXFP4 layers whose rows hold 4 k + 2 or 4 k + 3 steps of 64 elements, k from 0: the
+    grouped GEMMs' short last unit, in gate + up (N) and in down (M), on 32-entry tiles
+    (the first five; the fifth buckets in two blocks) and 64-entry tiles of one and two
+    entry blocks, with x in two fp16 planes and in one (bf16 values)."""
+    import torch
+    qts = (39, 39, 39)
+    rng = np.random.default_rng(N + M + T)
+    mats = [[W.gen_weights(rng, q, r, c) for _ in range(E)] for q, r, c in zip(qts, (M, M, N), (N, N, M))]
+    router, x = W.gen_router(rng, E, N), W.gen_x(rng, T, N, bf16=bf16)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    layer = dev.moe_prepare(qts, N, M, E, Kk, *[[cu(a) for a in m] for m in mats], cu(router), 1)
+    xt = cu(x)
+    got = layer.forward(xt).cpu().numpy()
+    ri, rw = orc.route(router, x, Kk, 1)
+    ref = np.stack([orc.moe_forward_token(*mats, x[t], M, N, qts, ri[t], rw[t]) for t in range(T)])
+    assert O.norm_err(got, ref) < moe_tol(qts)
+    for _ in range(20):
+        assert np.array_equal(layer.forward(xt).cpu().numpy(), got)
