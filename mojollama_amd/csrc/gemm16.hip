@@ -705,13 +705,18 @@ __global__ __launch_bounds__((64 * q16_wpg<SEM, DUAL, EB>()), (q16_waves<SEM, DU
             fw(s_beg + 1, rw[1]);
             fw(s_beg + 2, rw[2]);
         } else if constexpr (D == 3) {
+            // fenced on both sides: a weight load issued ahead of its step's activations would be
+            // one too many in the first step's count
             load_b(s_beg, std::integral_constant<int, 0>{});
+            __builtin_amdgcn_sched_barrier(0);
             fw(s_beg, rw[0]);
             __builtin_amdgcn_sched_barrier(0);
             load_b(s_beg + 1, std::integral_constant<int, 1>{});
+            __builtin_amdgcn_sched_barrier(0);
             fw(s_beg + 1, rw[1]);
             __builtin_amdgcn_sched_barrier(0);
             load_b(s_beg + 2, std::integral_constant<int, 2>{});
+            __builtin_amdgcn_sched_barrier(0);
             fw(s_beg + 2, rw[2]);
             __builtin_amdgcn_sched_barrier(0);
         } else {   // D == 1: step s issues the activations of s + 1 and the weights of s + 3
