@@ -7,7 +7,9 @@ the count of younger loads that may stay in flight is written in the source
 the order, and in the number, that it assumes.  A load too few, and a wave
 passes the barrier with a tile another wave reads still on its way: wrong
 results now and then.  So this follows every path through the built kernels and
-checks, at each step's barrier, that no load of that step is outstanding.
+checks, at each step's barrier, that no load of that step is outstanding, and
+that the wave's reads of the previous step's tile have returned (the loads that
+follow the barrier write over it).
 """
 import os
 import re
@@ -53,7 +55,8 @@ def listing(tmp_path_factory):
 
 def kernel_events(listing):
     """kernel -> (events, position by address): 'D' a load into LDS, 'V' another vector memory access, ('w', n) a
-    wait for all but the youngest n, 'B' a workgroup barrier, ('c' / 'j', target) a branch, 'E' the end."""
+    wait for all but the youngest n, 'R' an LDS access, 'L' a wait for all of them, 'B' a workgroup barrier,
+    ('c' / 'j', target) a branch, 'E' the end."""
     out = {}
     for name, body in re.findall(r"^[0-9a-f]+ <(_Z\S*5k_q16I\S*?)>:\n(.*?)(?=^\S|\Z)", listing, re.M | re.S):
         ev, at, base = [], {}, None
@@ -68,7 +71,11 @@ def kernel_events(listing):
                 ev.append("D")
             elif re.match(r"(buffer|global|flat|scratch)_(load|store|atomic)", op):
                 ev.append("V")
+            elif op.startswith("ds_"):
+                ev.append("R")
             elif op == "s_waitcnt":
+                if "lgkmcnt(0)" in arg:
+                    ev.append("L")
                 n = re.search(r"vmcnt\((\d+)\)", " ".join(arg))
                 if n:
                     ev.append(("w", int(n.group(1))))
@@ -89,7 +96,8 @@ def only_loads(ev, i, t):
 
 def faults(ev, at):
     """The barriers (0: the first step's, 1: the second's, 2: a later one's; with the loads a step and the steps
-    ahead) that some path reaches with a load of their step outstanding.
+    ahead) that some path reaches with a load of their step outstanding; "reads": a barrier of the main loop that
+    some path reaches with LDS reads outstanding.
 
     A state is a place in the code, the accesses that may be outstanding from the oldest load into LDS on, and how
     far the path is: the loads are numbered from 0, and from the second barrier on, which shows how many a step has,
@@ -98,18 +106,20 @@ def faults(ev, at):
     or three times that; a wave issues its loads in every step or in none."""
     bad, seen = set(), set()
     # place, outstanding, loads issued, barriers passed, loads a step (before the second barrier: at the first),
-    # loads ahead (before it: the oldest outstanding at the first), faults not yet counted
-    todo = [(0, (), 0, 0, 0, -1, ())]
+    # loads ahead (before it: the oldest outstanding at the first), faults not yet counted, LDS reads outstanding
+    todo = [(0, (), 0, 0, 0, -1, (), False)]
     while todo:
         st = todo.pop()
         while st not in seen:
             seen.add(st)
-            i, q, n, nb, per, low, f = st
+            i, q, n, nb, per, low, f, r = st
             e, i = ev[i], i + 1
             if e == "D":
                 q, n = q + (n,), n + 1
             elif e == "V":
                 q = q + ("V",) if q else q
+            elif e == "R" or e == "L":
+                r = e == "R"
             elif e == "E":
                 break
             elif e == "B":
@@ -127,6 +137,7 @@ def faults(ev, at):
                     if n - per != low:
                         break
                     bad |= set(f) | ({(2, per, low // per + 1)} if low_now < per else set())
+                    bad |= {"reads"} if r else set()
                     q, n = tuple(k if k == "V" else k - per for k in q), n - per
                     f = ()
             elif e[0] == "w":
@@ -140,8 +151,8 @@ def faults(ev, at):
                 # them in every step; those that issue them have something to wait for
                 t = at[e[1]]
                 if not only_loads(ev, i, t):
-                    todo.append((t, q, n, nb, per, low, f))
-            st = (i, q, n, nb, per, low, f)
+                    todo.append((t, q, n, nb, per, low, f, r))
+            st = (i, q, n, nb, per, low, f, r)
     return bad
 
 
