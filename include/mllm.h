@@ -226,7 +226,8 @@ MLLM_API int mllm_pack(int sem, const void *raw_dev, void *packed_dev, int n_row
  * At 2 <= B <= 8 the Q4_K, Q6_K, Q8_0, Q4_0 and MXFP4 batch semantics run on
  * the matrix cores from the batch where that is faster; given the workspace,
  * short matrices there also split K over more workgroups (optional: NULL
- * runs unsplit or on the vector kernel). */
+ * runs unsplit or on the vector kernel).  A workspace sized for B serves every
+ * smaller batch of the same matrix (the size never decreases with B). */
 MLLM_API long mllm_gemv_workspace_size(int sem, int n_rows, int n_cols, int B);
 MLLM_API int mllm_gemv(int sem, const void *packed_dev, const float *x_dev, float *out_dev, int n_rows, int n_cols,
                        int B, void *workspace, void *stream);
@@ -247,7 +248,8 @@ MLLM_API int mllm_gemv(int sem, const void *packed_dev, const float *x_dev, floa
  * x_up excludes x_res/res_out/rms_w and silu_pair.  Shapes the decode kernel
  * can stage at once (B <= 8; paired rows at B == 1) run as one launch; others
  * form the activation in the workspace first and the SiLU product after the
- * GEMV (mllm_gemv_fused_workspace_size bytes). */
+ * GEMV (mllm_gemv_fused_workspace_size bytes, which serve every smaller batch
+ * of the same matrix and fusion too). */
 typedef struct {
     const float *x_up;
     int silu_clamp;

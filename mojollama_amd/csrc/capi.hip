@@ -527,6 +527,21 @@ size_t gemv_scratch_bytes(int sem, int n_rows, int n_cols, int B)
     return std::max(gemv_required_bytes(sem, n_rows, n_cols, B), gemv_mf_bytes(sem, n_rows, n_cols, B));
 }
 
+// The largest need(b) over the batches b <= B, so that a workspace serves every smaller batch
+// too (the launches split K more the fewer tokens there are: Q4_K 3072 x 2048 needs 6.9 MB at
+// 64 tokens, 2.2 MB at 65).  need grows with the batch except where the kernel, the entry tiles or
+// their size change: after 1 .. 8, at multiples of 64, and at 256 and 512.  From 49152 tokens on
+// (384 tiles of 128 entries) nothing is split.
+template <class F> size_t max_over_batches(int B, F need)
+{
+    size_t m = need(B);
+    for (int b = 1; b < std::min(B, 9); b++) m = std::max(m, need(b));
+    for (int b : {255, 511})
+        if (b < B) m = std::max(m, need(b));
+    for (int b = 64; b < B && b <= 49152; b += 64) m = std::max(m, need(b));
+    return m;
+}
+
 // Queue GEMV(s) over B tokens (any B: split into groups of 8) on device data;
 // out_add (optional, same layout as out; on the bf16-tile GEMM not overlapping
 // it, on the fp16-plane GEMM equal to it or apart) is added to the result.
@@ -1046,7 +1061,7 @@ MLLM_API int mllm_pack(int sem, const void *raw_dev, void *packed_dev, int n_row
 
 MLLM_API long mllm_gemv_workspace_size(int sem, int n_rows, int n_cols, int B)
 {
-    return (long)gemv_scratch_bytes(sem, n_rows, n_cols, B);
+    return (long)max_over_batches(B, [&](int b) { return gemv_scratch_bytes(sem, n_rows, n_cols, b); });
 }
 
 MLLM_API int mllm_gemv(int sem, const void *packed_dev, const float *x_dev, float *out_dev, int n_rows, int n_cols,
@@ -1106,7 +1121,7 @@ static fused_ws fused_layout(int sem, int n_rows, int n_cols, int B, const mllm_
 MLLM_API long mllm_gemv_fused_workspace_size(int sem, int n_rows, int n_cols, int B, const mllm_gemv_fusion *f)
 {
     if (sem < 0 || sem >= SEM_COUNT || B <= 0) return -1;
-    return (long)fused_layout(sem, n_rows, n_cols, B, f).total;
+    return (long)max_over_batches(B, [&](int b) { return fused_layout(sem, n_rows, n_cols, b, f).total; });
 }
 
 MLLM_API int mllm_gemv_fused(int sem, const void *packed_dev, const float *x_dev, float *out_dev, int n_rows,

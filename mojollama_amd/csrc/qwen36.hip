@@ -428,7 +428,7 @@ void mllm_qwen36_cache_clear()
 
 namespace {
 
-// Per-call buffers for B tokens.
+// Per-call buffers for B tokens (kept for smaller batches: no size query decreases with B).
 int q36_buffers(q36_model &m, int B)
 {
     if (B <= m.B_cap) return 0;

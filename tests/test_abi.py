@@ -131,3 +131,21 @@ def test_attention_rejects_bad_strides(libpath):
     kv = kernels.KVView(fake, fake, 64, None, 0, 0, 0)
     assert so.mllm_kv_append(ctypes.byref(kv), fake, fake, fake, 2, 2, 64, None) == -1
     assert b"seq_stride" in so.mllm_last_error()
+
+
+@pytest.mark.parametrize("rows,cols", [(3072, 2048), (5632, 2048), (2048, 5632), (32000, 2048), (11264, 4096), (1000, 9216),
+                                       (128, 256), (1, 32)])
+def test_gemv_workspace_never_decreases_with_the_batch(libpath, rows, cols):
+    """mllm_gemv and mllm_gemv_fused take no workspace size: one sized for the largest
+    batch has to serve the smaller ones (qwen36_batch_forward keeps its own like that)."""
+    from mojollama_amd import kernels as K
+    so = K.load_kernels()
+    p = 256                                       # any non-null vector: the sizes do not read it
+    fusions = [K.GemvFusion(), K.GemvFusion(out_add=p), K.GemvFusion(rms_w=p, x_res=p, res_out=p), K.GemvFusion(x_up=p),
+               K.GemvFusion(silu_pair=1, rms_w=p)]
+    for sem in (K.Q4_K_GGML, K.Q6_K_SEQ, K.Q6_K_LOWNIB, K.Q4_K_Q8, K.Q8_0, K.Q4_0, K.MXFP4, K.MXFP4_Q8):
+        sizes = [[so.mllm_gemv_workspace_size(sem, rows, cols, b) for b in range(1, 1100)]]
+        sizes += [[so.mllm_gemv_fused_workspace_size(sem, rows, cols, b, ctypes.byref(f)) for b in range(1, 1100)]
+                  for f in fusions]
+        for n in sizes:
+            assert all(a <= b for a, b in zip(n, n[1:])), (K.SEM_NAMES[sem], rows, cols)
