@@ -844,7 +844,7 @@ bool mllm_qgemm_supported(int sem)
 // than 8).
 int mllm_qgemm_ksplit(int sem, int n_rows, int n_cols, int n_entries)
 {
-    if (!mllm_qgemm_supported(sem) || n_entries <= 0) return 1;
+    if (!mllm_qgemm_supported(sem) || n_rows <= 0 || n_entries <= 0) return 1;
     const int tm = (n_entries >= 512 && sem != SEM_Q4_K_Q8 && sem != SEM_MXFP4_Q8) ? 128 : 64;
     const long tiles = (long)((n_rows + 127) / 128) * ((n_entries + tm - 1) / tm);
     if (tiles >= 256) return 1;

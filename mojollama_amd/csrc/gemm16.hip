@@ -1518,7 +1518,7 @@ int mllm_q16_tile_entries(bool grouped, int n_entries) { return !grouped && n_en
 // -> 24.5, 32000 x 2048 38.9 -> 46.4).
 int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries)
 {
-    if (!mllm_q16_supported(sem) || n_entries <= 0) return 1;   // MXFP4: grouped launches, no split
+    if (!mllm_q16_supported(sem) || n_rows <= 0 || n_entries <= 0) return 1;   // MXFP4: grouped launches, no split
     const int tm = mllm_q16_tile_entries(false, n_entries);
     const long tiles = (long)((n_rows + 127) / 128) * ((n_entries + tm - 1) / tm);
     if (tiles >= 384) return 1;

@@ -4,6 +4,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -149,3 +150,10 @@ def test_gemv_workspace_never_decreases_with_the_batch(libpath, rows, cols):
                   for f in fusions]
         for n in sizes:
             assert all(a <= b for a, b in zip(n, n[1:])), (K.SEM_NAMES[sem], rows, cols)
+
+
+def test_gemv_workspace_of_no_rows(libpath):
+    """A matrix without rows has no output tile to split (no division by their number)."""
+    code = ("from mojollama_amd import kernels as K; so = K.load_kernels()\n"
+            "assert all(so.mllm_gemv_workspace_size(s, 0, 2048, b) >= 0 for s in range(16) for b in (1, 8, 32, 300))")
+    assert subprocess.run([sys.executable, "-c", code], cwd=ROOT).returncode == 0
