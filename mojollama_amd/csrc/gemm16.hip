@@ -275,12 +275,12 @@ MLLM_DEV void q16_min_mk(const q16_min_raw &r, int nb, int u0, f16x8 &hi, f16x8 
             v[j] = live ? -(dmin * (float)m1) : 0.0f;
             v[j + 1] = live ? -(dmin * (float)m2) : 0.0f;
         }
+        // (without split16's select for infinities, which activations need: every dense Q4_K
+        // launch runs this, 5632 x 2048 at 1280 tokens 82.3 us with it, 82.0 without)
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            _Float16 a, c;
-            split16(v[j], a, c);
-            hi[j] = a;
-            lo[j] = c;
+            hi[j] = (_Float16)v[j];
+            lo[j] = (_Float16)(v[j] - (float)hi[j]);
         }
     } else {
         const uint32_t w[8] = {r.m.x, r.m.y, r.m.z, r.m.w, r.m2.x, r.m2.y, r.m2.z, r.m2.w};
