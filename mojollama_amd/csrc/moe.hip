@@ -340,11 +340,12 @@ static int moe_q16_setup(mllm_moe_layer *L)
     return 0;
 }
 
-// Tokens up to which other layers run the decode GEMVs (one job per (token,
-// slot); an expert picked by several tokens is streamed once per token) rather
-// than the bucketed grouped GEMMs.  Measured on MI355X: GPT-OSS shape 225 vs
-// 388 us at T = 16, 407 vs 385 us at T = 32; Qwen3 shape 119 vs 256 us at
-// T = 16, 219 vs 312 us at T = 32, 358 vs 342 us at T = 64.
+// Tokens past which every layer runs the bucketed grouped GEMMs rather than the decode GEMVs (one
+// job per (token, slot); an expert picked by several tokens is streamed once per token).  The
+// GEMVs lead at 24 in each layer measured that moe_grouped does not hand over earlier; where they
+// fall behind differs, GEMV / grouped in us at T = 24 and 32: Q6_K 2560 x 1536, 32 experts, top 4
+// 208 / 226, 273 / 243; 1024 x 1024, 8, 4 69 / 78, 91 / 78; Q4_0 2048 x 768, 128, 8 145 / 326,
+// 186 / 356; MXFP4 2848 x 2848, 32, 4 (no whole 64-column steps) 288 / 447, 398 / 452.
 constexpr int kMoeDecodeMaxT = 24;
 
 // Layers whose gate/up and down both run on the fp16-plane GEMM with 32-entry tiles.
@@ -365,19 +366,34 @@ static bool moe_tile32(const mllm_moe_layer &L, int T)
     return moe_q16_small(L) && TK <= 24L * L.E && TK * L.M >= 3 * (TK / 32 + L.E + 1) + 1;
 }
 
-// Whether T tokens run the bucketed grouped GEMMs.  Layers on 32-entry tiles take them from
-// the T where streaming each picked expert once (expected number E (1 - (1 - K/E)^T)) costs
-// less than streaming it per token: GEMVs 18 us + bytes at 4.5 TB/s, grouped 45 us + bytes at
-// 2.9 TB/s, fitted to, GEMV / grouped: GPT-OSS T = 8 117 / 127 us, 12 166 / 140, 16 211 / 177,
-// 24 290 / 185; Qwen3 T = 16 103 / 115, 24 135 / 144, 32 175 / 153.
+// Whether T tokens run the bucketed grouped GEMMs.  Layers on 32-entry tiles take them below
+// kMoeDecodeMaxT where an estimate of their time is the shorter one by a twentieth.  The GEMVs
+// stream every picked expert once per token: 28 us and the bytes at 4.1 TB/s in MXFP4, 6.0 in
+// Q4_K / Q6_K.  The grouped launches' time is chains of steps: 40 us, and per 256 columns of a
+// matrix so much and again so much for each workgroup (128 rows of one of the expected
+// E (1 - (1 - K/E)^T) picked experts) that a CU runs beside its first.  Constants fitted to 300
+// timings of 70 layers (MXFP4 of 512 .. 2880 columns, 8 .. 64 experts, top 2 .. 6; Q4_K / Q6_K of
+// 512 .. 2560, 8 .. 128 experts, top 2 .. 8; T = 9 .. 24; estimates within 5 % and 8 % rms).  Where
+// the rule takes the GEMMs they ran 0.96 to 5.2 times as fast, GEMV / grouped in us: GPT-OSS
+// (2880 x 2880, 32 experts, top 4) T = 16 216 / 181, 24 293 / 182; 2752 x 1216, 14, 6, T = 9 102 /
+// 82; Q4_K 2560 x 1024, 9, 6, T = 14 99 / 75; where it does not: GPT-OSS T = 12 170 / 176; 1536 x
+// 1536, 8, 2, T = 24 58 / 61; Qwen3 (2048 x 768, 128, 8) T = 24 135 / 141; Q4_K 1024 x 1024, 8, 4,
+// T = 24 49 / 57; 2560 x 1536, 16, 2, T = 24 80 / 87.
 static bool moe_grouped(const mllm_moe_layer &L, int T)
 {
     if (T > kMoeDecodeMaxT) return true;
     if (T <= 8 || !moe_tile32(L, T)) return false;
-    const double mb = 1e-6 * (2.0 * mllm_packed_bytes(mllm_sem_layout(L.sem_g), L.M, L.N, nullptr) +
-                              (double)mllm_packed_bytes(mllm_sem_layout(L.sem_d), L.N, L.M, nullptr));
     const double picked = L.E * (1.0 - std::pow(1.0 - (double)L.K / L.E, T));
-    return 45.0 + picked * mb / 2.9 < 18.0 + (double)T * L.K * mb / 4.5;
+    double gemv = 28.0, grouped = 40.0;
+    auto half = [&](int sem, int rows, int cols, int mats, double first_mx, double each_mx, double first, double each) {
+        const bool mx = mllm_q16_mx(sem);
+        const double per_cu = std::ceil((rows + 127) / 128 * picked / 256.0);
+        gemv += 1e-6 * T * L.K * mats * mllm_packed_bytes(mllm_sem_layout(sem), rows, cols, nullptr) / (mx ? 4.1 : 6.0);
+        grouped += cols / 256.0 * (mx ? first_mx + each_mx * per_cu : first + each * per_cu);
+    };
+    half(L.sem_g, L.M, L.N, 2, 1.2, 2.2, 0.9, 1.7);
+    half(L.sem_d, L.N, L.M, 1, 0.0, 1.2, 0.0, 2.5);
+    return 1.05 * grouped < gemv;
 }
 
 static size_t moe_ws_layout(const mllm_moe_layer &L, int T, moe_ws *w, uint8_t *base)

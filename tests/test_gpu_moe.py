@@ -568,23 +568,27 @@ def test_moe_forward_omp_empty_slots(lib, orc):
 @pytest.mark.parametrize("qts,N,M,E,Kk,T", [
     ((39, 39, 39), 1024, 1024, 8, 4, 20), ((39, 39, 39), 960, 1088, 8, 4, 24), ((12, 12, 14), 1024, 1024, 8, 4, 24),
     ((39, 39, 39), 192, 320, 20, 3, 100), ((12, 12, 14), 512, 256, 8, 2, 96), ((12, 12, 14), 256, 512, 16, 1, 40),
-    ((39, 39, 39), 64, 64, 256, 1, 25), ((39, 39, 39), 128, 128, 30, 4, 400)])
+    ((39, 39, 39), 64, 64, 256, 1, 25), ((39, 39, 39), 128, 128, 30, 4, 400), ((39, 39, 39), 1024, 2048, 8, 8, 9),
+    ((39, 39, 39), 960, 1088, 8, 8, 24), ((12, 12, 14), 1024, 1024, 8, 8, 24), ((12, 12, 14), 768, 1024, 12, 8, 17),
+    ((39, 39, 39), 512, 256, 64, 4, 300)])
 def test_moe_layer_32_entry_tiles(dev, orc, qts, N, M, E, Kk, T):
-    """Few entries per expert: the grouped GEMMs on 32-entry tiles, from 9
-    tokens where streaming each picked expert once is cheaper (the first three),
-    with experts of more than 32 entries (one to three tiles) and of none, ragged
-    last rows of a 128-row tile, step counts that are no multiple of four, and
-    the bucketing by one block and by two (1600 entries)."""
+    """Few entries per expert: the grouped GEMMs on 32-entry tiles, from 9 tokens where
+    their estimate is the shorter (top 8 of 8 and of 12; the first three, top 4 of 8, lie
+    near that line), with experts of more than 32 entries (one to three tiles) and of none,
+    ragged last rows of a 128-row tile, step counts that are no multiple of four, and the
+    bucketing by one block and by two (1200 entries; 1600 over 30 experts take 64-entry
+    tiles)."""
     got, ref = _moe_case(dev, orc, qts, N=N, M=M, E=E, Kk=Kk, T=T, renorm=T % 2, seed=T + N + M)
     assert O.norm_err(got, ref) < moe_tol(qts)
 
 
 @pytest.mark.parametrize("qts", [(39, 39, 39), (12, 12, 14)])
-def test_moe_layer_32_entry_tiles_nonfinite_token(dev, orc, qts):
+@pytest.mark.parametrize("Kk", [4, 8])
+def test_moe_layer_32_entry_tiles_nonfinite_token(dev, orc, qts, Kk):
     """A token with an infinite element is routed to no expert (zeros); the others are untouched."""
     import torch
     rng = np.random.default_rng(81)
-    N, M, E, Kk, T = 1024, 1024, 8, 4, 24
+    N, M, E, T = 1024, 1024, 8, 24
     mats = [[W.gen_weights(rng, q, r, c) for _ in range(E)] for q, r, c in zip(qts, (M, M, N), (N, N, M))]
     router, x = W.gen_router(rng, E, N), W.gen_x(rng, T, N)
     x[3, 17] = np.inf
