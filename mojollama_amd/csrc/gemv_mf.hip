@@ -36,19 +36,24 @@ int mf_block(int sem) { return (sem == SEM_Q4_K_GGML || sem == SEM_Q6_K_SEQ) ? 2
 
 // Rows short enough that a workgroup stages all of them in one or two passes and each wave
 // has few units stay whole: a split saves little there, and the launch that joins it costs
-// more.  Four blocks and a head of 1024 rows, B = 8, split / whole: N = 1024 Q4_K 172.7 /
-// 150.4 us, Q8_0 200.6 / 176.3, MXFP4 179.5 / 171.0, Q4_0 175.9 / 143.4; N = 2048 Q4_K 216.9 /
-// 211.0, Q4_0 200.0 / 200.1, but MXFP4 215.5 / 222.3 and Q8_0 234.3 / 240.0; 4096 columns of
-// Q4_K, B = 3, 246.5 / 252.9.  Fewer than 32 tiles (an eighth of the CUs) were not tried.
-constexpr int kMfWholeTiles = 32;
-int mf_whole_cols(int sem)
+// more.  One matrix from a graph, split / whole in us: 256 rows, B = 8, of 512 columns Q4_K
+// 5.7 / 4.1, Q6_K 7.5 / 5.8, Q8_0 8.3 / 6.1, Q4_0 7.5 / 4.7, MXFP4 7.3 / 4.2; of 1536 7.1 / 6.3,
+// 8.8 / 8.3, 8.7 / 8.6, 7.7 / 6.8, 7.4 / 6.9; of 2048 7.9 / 7.3, 9.6 / 9.2, 8.9 / 8.9, 7.9 / 8.1,
+// 8.1 / 8.1 (B = 5: MXFP4 8.1 / 9.2); of 2304 7.8 / 8.2, 9.2 / 10.1, -, 7.4 / 8.5, -.  From 32 tiles of
+// rows on the split has more to join: 1536 rows of 2304 columns Q4_K 10.3 / 9.1, Q6_K 11.4 / 11.3,
+// Q4_0 9.9 / 8.6, but MXFP4 and Q8_0 of 2048 as before 10.9 / 10.9, 13.3 / 13.5.  Whole decode
+// passes of 2048 columns, B = 8: MXFP4 215.5 / 222.3, Q8_0 234.3 / 240.0; 4096 columns of Q4_K,
+// B = 3, 246.5 / 252.9.
+int mf_whole_cols(int sem, int n_tiles)
 {
-    return sem == SEM_Q4_K_GGML || sem == SEM_Q6_K_SEQ || sem == SEM_Q4_0 ? 2304 : 1536;
+    const bool kq = sem == SEM_Q4_K_GGML || sem == SEM_Q6_K_SEQ;
+    if (n_tiles >= 32 && (kq || sem == SEM_Q4_0)) return 2304;
+    return kq ? 2048 : 1536;
 }
 
 // S: the fewest K splits whose range fits the LDS budget, raised (up to 8
 // and one 256-element block per split) until rows x splits give a tile per
-// CU (but see kMfWholeTiles); without a partials buffer only S = 1.
+// CU (but see mf_whole_cols); without a partials buffer only S = 1.
 mf_plan mf_plan_for(int sem, int n_rows, int n_cols, int B, bool pro, bool pair, bool have_part)
 {
     mf_plan p{};
@@ -66,7 +71,7 @@ mf_plan mf_plan_for(int sem, int n_rows, int n_cols, int B, bool pro, bool pair,
     const int smax = std::min(nb, kMfMaxSplits);
     while (S < smax && lds_for(S) > (size_t)kMfLdsCap) S++;
     if (lds_for(S) > (size_t)kMfLdsCap) return p;
-    if (S > 1 || p.n_tiles < kMfWholeTiles || n_cols > mf_whole_cols(sem))
+    if (S > 1 || n_cols > mf_whole_cols(sem, p.n_tiles))
         while (S < smax && (long)p.n_tiles * S < cus) S++;
     if (!have_part) {
         if (lds_for(1) > (size_t)kMfLdsCap) return p;

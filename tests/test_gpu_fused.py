@@ -242,9 +242,11 @@ def test_fused_prologue_kernel_rows(dev, orc, C, ld, B):
 
 @pytest.mark.parametrize("sem,R,C,B", [(K.Q4_K_GGML, 993, 2304, 8), (K.Q4_K_GGML, 992, 2304, 8),
                                        (K.Q4_K_GGML, 1024, 2560, 8), (K.Q6_K_SEQ, 1056, 1280, 3),
-                                       (K.Q8_0, 1001, 1536, 7), (K.MXFP4, 1024, 1568, 5), (K.MXFP4, 993, 32, 8)])
+                                       (K.Q8_0, 1001, 1536, 7), (K.MXFP4, 1024, 1568, 5), (K.MXFP4, 993, 32, 8),
+                                       (K.Q4_K_GGML, 257, 2048, 5), (K.Q6_K_SEQ, 33, 2048, 8), (K.Q4_0, 100, 1536, 6),
+                                       (K.Q4_0, 100, 1568, 6), (K.Q8_0, 31, 1536, 8), (K.Q6_K_SEQ, 70, 2304, 4)])
 @pytest.mark.parametrize("mode", ["rms", "rms_div_res", "res_add", "add_inplace"])
 def test_fused_mf_whole_rows(dev, orc, sem, R, C, B, mode):
-    """B = 2..8 on the matrix cores at the edge between whole rows (32 tiles
-    of 32 rows and up, columns to the type's limit) and a split along K."""
+    """B = 2..8 on the matrix cores at the edge between whole rows (columns to
+    the type's limit, a longer one from 32 tiles of 32 rows on) and a split along K."""
     run_case(dev, orc, sem, R, C, B, mode, seed=R + C + B + len(mode))
