@@ -573,7 +573,7 @@ int run_gemv(int sem, const mllm_packed &W, const float *x, float *out, int n_ro
         g.out = out; g.ldo = pair ? n_rows / 2 : n_rows;
         g.add = out_add; g.pair = pair; g.clamp_silu = clamp;
         g.n_rows = n_rows; g.n_cols = n_cols; g.n_entries = B;
-        g.ksplit = mllm_q16_ksplit(sem, n_rows, n_cols, B);
+        g.ksplit = mllm_q16_ksplit(sem, n_rows, n_cols, B, pro || out_add || pair);
         if (g.ksplit > 1) g.part = (float *)ws;
         HIP_OK(mllm_launch_q16(sem, false, g, 0, st));
         return 0;
@@ -1203,7 +1203,7 @@ MLLM_API int mllm_gemv_fused(int sem, const void *packed_dev, const float *x_dev
         set_error("mllm_gemv_fused: a strided x (x_ld) needs a fused activation step on this path");
         return -1;
     }
-    if (pair && q16 && mllm_q16_ksplit(sem, mrows, n_cols, B) > 1)
+    if (pair && q16 && mllm_q16_ksplit(sem, mrows, n_cols, B, true) > 1)
         // gate, up and the SiLU product joined from the split's partial sums
         return run_gemv(sem, view, xa, out_dev, mrows, n_cols, B, ws + L.gemv, st, out_add, true, pro16 ? &p16 : nullptr,
                         ldx, true, f->silu_clamp != 0);

@@ -127,10 +127,12 @@ struct q16_args {
 bool mllm_q16_tile32(int sem, bool dual);
 // Entries per work tile of a launch (grouped launches: the bucketing's tile).
 int mllm_q16_tile_entries(bool grouped, int n_entries);
-int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries);
+// The splits of a dense launch (fused: with a prologue, a residual or paired rows) and the
+// floats of its partial sums (for either form; a fused launch splits wherever a plain one does).
+int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries, bool fused);
 inline long mllm_q16_part_floats(int sem, int n_rows, int n_cols, int n_entries)
 {
-    const int ks = mllm_q16_ksplit(sem, n_rows, n_cols, n_entries);
+    const int ks = mllm_q16_ksplit(sem, n_rows, n_cols, n_entries, true);
     return ks > 1 ? (long)ks * n_entries * n_rows : 0;
 }
 hipError_t mllm_launch_q16(int sem, bool dual, const q16_args &a, int max_tiles, hipStream_t st);

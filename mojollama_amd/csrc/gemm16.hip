@@ -1515,18 +1515,25 @@ int mllm_q16_tile_entries(bool grouped, int n_entries) { return !grouped && n_en
 // (rows x K at 32 tokens, staging and join included, at least 4 super-blocks
 // each against at least 1: 2560 x 2048 21.7 -> 16.4 us, 2048 x 5632 36.9 ->
 // 23.7; at least 2: 17.8 and 25.2; 768 workgroups for 512: 11264 x 2048 23.0
-// -> 24.5, 32000 x 2048 38.9 -> 46.4).
-int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries)
+// -> 24.5, 32000 x 2048 38.9 -> 46.4).  The exception: plain calls of Q4_K rows of
+// two super-blocks at up to 32 tokens.  The one saved is worth less than queueing
+// a third launch (whole / split, 10 tokens: 512 x 512 12.3 / 14.6, 8192 x 512 12.3 /
+// 14.5; 64 tokens 14.9 / 14.6; three super-blocks, 512 x 768, 10 tokens 14.8 / 14.3;
+// Q6_K of two 15.1 / 14.4).  Fused calls, as in a captured decode pass, split there
+// too (four 512-column blocks and a head, 32 tokens, 281.6 / 274.5).
+int mllm_q16_ksplit(int sem, int n_rows, int n_cols, int n_entries, bool fused)
 {
     if (!mllm_q16_supported(sem) || n_rows <= 0 || n_entries <= 0) return 1;   // MXFP4: grouped launches, no split
     const int tm = mllm_q16_tile_entries(false, n_entries);
     const long tiles = (long)((n_rows + 127) / 128) * ((n_entries + tm - 1) / tm);
     if (tiles >= 384) return 1;
     const int nb = n_cols / 256;
-    if (n_entries <= 64) return std::max(1, std::min({(int)(512 / tiles), nb, 32}));
     int ks = (int)(512 / tiles);
-    ks = std::min(ks, std::max(1, nb / 4));
-    return std::max(1, std::min(ks, 8));
+    ks = n_entries <= 64 ? std::min({ks, nb, 32}) : std::min({ks, std::max(1, nb / 4), 8});
+    const bool q4k = sem == SEM_Q4_K_GGML || sem == SEM_Q4_K_Q8;
+    if (ks <= 1 || (q4k && nb <= 2 && n_entries <= 32 && !fused)) return 1;
+    const int each = (nb + ks - 1) / ks;   // super-blocks of a split (k_q16)
+    return (nb + each - 1) / each;         // the splits they fill
 }
 
 hipError_t mllm_launch_q16(int sem, bool dual, const q16_args &a, int max_tiles, hipStream_t st)

@@ -178,19 +178,22 @@ def test_fused_silu_pair(dev, orc, sem, C, B, mode):
 
 @pytest.mark.parametrize("sem,R,C,B", [(K.Q4_K_GGML, 303, 2048, 9), (K.Q6_K_SEQ, 130, 5632, 33),
                                        (K.Q4_K_GGML, 2048, 256, 64), (K.Q6_K_SEQ, 516, 9216, 11),
-                                       (K.Q4_K_GGML, 4100, 512, 300), (K.Q4_K_Q8, 300, 2048, 40)])
+                                       (K.Q4_K_GGML, 4100, 512, 300), (K.Q4_K_Q8, 300, 2048, 40),
+                                       (K.Q4_K_GGML, 260, 512, 32), (K.Q4_K_GGML, 259, 512, 33), (K.Q4_K_Q8, 100, 512, 9),
+                                       (K.Q6_K_SEQ, 131, 512, 10), (K.Q4_K_GGML, 11264, 2304, 20)])
 @pytest.mark.parametrize("mode", ["rms", "rms_div_res", "res_add", "add_inplace", "silu"])
 def test_fused_batched(dev, orc, sem, R, C, B, mode):
     """B > 8 on the fp16-plane GEMM: the prologue formed while the activation
     is staged (rows up to 8192; 9216 takes the separate launch), K split down
-    to one super-block per workgroup, the residual added in the join of the
+    to one super-block per workgroup (Q4_K rows of two whole up to 32 tokens; 9 over
+    two each: the last split holds one), the residual added in the join of the
     partial sums or, unsplit, in the GEMM's own epilogue."""
     run_case(dev, orc, sem, R, C, B, mode, seed=R + C + B + len(mode))
 
 
 @pytest.mark.parametrize("sem,R,C,B", [(K.Q4_K_GGML, 150, 2048, 9), (K.Q4_K_GGML, 301, 512, 65),
                                        (K.Q6_K_LOWNIB, 96, 768, 33), (K.Q4_K_Q8, 128, 1024, 17),
-                                       (K.Q4_K_GGML, 24580, 256, 10)])
+                                       (K.Q4_K_GGML, 24580, 256, 10), (K.Q4_K_GGML, 130, 512, 16)])
 @pytest.mark.parametrize("mode", ["pair", "pair_rms", "pair_noclamp_add"])
 def test_fused_silu_pair_batched(dev, orc, sem, R, C, B, mode):
     """Paired rows at B > 8: the SiLU product in the join of the split's
