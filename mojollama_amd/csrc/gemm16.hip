@@ -1014,9 +1014,7 @@ __global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int 
     }
     if (TPR < 256 && row >= rows) return;
     const float *xr = x + (long)row * ldx;
-    // 16-byte loads where every vector the prologue reads allows them
-    const bool vec = (((uintptr_t)xr | (PRO && pro.x_up ? (uintptr_t)(pro.x_up + (long)row * ldx) : 0) |
-                       (PRO && pro.x_res ? (uintptr_t)(pro.x_res + (long)row * ldx) : 0)) & 15) == 0;
+    const bool vec = ((uintptr_t)xr & 15) == 0;
     const int nb = K / Q::EPS;
     // eight consecutive elements from k (a multiple of 8)
     auto ld8 = [&](int k, float (&v)[8]) __attribute__((always_inline)) {
