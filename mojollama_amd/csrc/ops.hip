@@ -793,15 +793,17 @@ __global__ void k_silu_mul(const float *__restrict__ g, const float *__restrict_
 // stays in registers between the two passes (kProHeld groups of V elements a
 // thread, all loads issued at once; longer rows loop over it through out): a
 // token's row is one workgroup's work, so its time is memory latencies -- one
-// row of 2880 elements 9.4 -> 2.8 us against 256 threads looping twice.
+// row of 2880 elements 9.4 -> 2.8 us with 1024 threads against 256 looping
+// twice.  Rows that 256 threads hold in one group take 256: of more, most would
+// wait for the rest (1280 rows of 512 elements 7.7 us with 1024 threads, 4.3 with 256).
 constexpr int kProThreads = 1024, kProHeld = 4;
-template <int V, bool HELD>
-__global__ __launch_bounds__(kProThreads) void k_act_prologue(const float *__restrict__ x, const float *__restrict__ x_res,
-                                                              float *__restrict__ res_out, const float *__restrict__ rms_w,
-                                                              float eps, int div, const float *__restrict__ x_up, int clamp,
-                                                              int n, int ldx, float *__restrict__ out)
+template <int V, bool HELD, int TH>
+__global__ __launch_bounds__(TH) void k_act_prologue(const float *__restrict__ x, const float *__restrict__ x_res,
+                                                     float *__restrict__ res_out, const float *__restrict__ rms_w,
+                                                     float eps, int div, const float *__restrict__ x_up, int clamp,
+                                                     int n, int ldx, float *__restrict__ out)
 {
-    __shared__ float red[kProThreads / 64];
+    __shared__ float red[TH / 64];
     const long xo = (long)blockIdx.x * ldx, o = (long)blockIdx.x * n;
     const int tid = threadIdx.x;
     typedef float vf __attribute__((ext_vector_type(V)));
@@ -827,23 +829,23 @@ __global__ __launch_bounds__(kProThreads) void k_act_prologue(const float *__res
     if constexpr (HELD) {
 #pragma unroll
         for (int k = 0; k < kProHeld; k++) {
-            const int i = V * (tid + kProThreads * k);
+            const int i = V * (tid + TH * k);
             if (i < n) h[k] = form(i);
         }
 #pragma unroll
         for (int k = 0; k < kProHeld; k++) {
-            const int i = V * (tid + kProThreads * k);
+            const int i = V * (tid + TH * k);
             if (i < n) put(i, h[k]);
         }
     } else {
-        for (int i = V * tid; i < n; i += V * kProThreads) put(i, form(i));
+        for (int i = V * tid; i < n; i += V * TH) put(i, form(i));
     }
     if (!rms_w) return;
     for (int d = 32; d >= 1; d >>= 1) ss += __shfl_xor(ss, d, 64);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
-    ss = red[tid & (kProThreads / 64 - 1)];
-    for (int d = kProThreads / 128; d >= 1; d >>= 1) ss += __shfl_xor(ss, d, 64);
+    ss = red[tid & (TH / 64 - 1)];
+    for (int d = TH / 128; d >= 1; d >>= 1) ss += __shfl_xor(ss, d, 64);
     const float r = sqrtf(ss / (float)n + eps);
     const float sc = div ? r : 1.0f / r;
     auto norm = [&](int i, vf v) __attribute__((always_inline)) {
@@ -855,11 +857,11 @@ __global__ __launch_bounds__(kProThreads) void k_act_prologue(const float *__res
     if constexpr (HELD) {
 #pragma unroll
         for (int k = 0; k < kProHeld; k++) {
-            const int i = V * (tid + kProThreads * k);
+            const int i = V * (tid + TH * k);
             if (i < n) norm(i, h[k]);
         }
     } else {
-        for (int i = V * tid; i < n; i += V * kProThreads) norm(i, ld(out + o + i));   // written by this same thread above
+        for (int i = V * tid; i < n; i += V * TH) norm(i, ld(out + o + i));   // written by this same thread above
     }
 }
 
@@ -1150,13 +1152,19 @@ hipError_t mllm_launch_act_prologue(const float *x, const float *x_res, float *r
     const bool v4 = n % 4 == 0 && ldx % 4 == 0 &&
                     (((uintptr_t)x | (uintptr_t)x_res | (uintptr_t)res_out | (uintptr_t)rms_w | (uintptr_t)x_up |
                       (uintptr_t)out) & 15) == 0;
-    const bool held = n <= kProThreads * kProHeld * (v4 ? 4 : 1);
-    auto go = [&](auto v_c, auto h_c) {
-        hipLaunchKernelGGL((k_act_prologue<decltype(v_c)::value, decltype(h_c)::value>), dim3(T), dim3(kProThreads), 0,
-                           st, x, x_res, res_out, rms_w, eps, div, x_up, clamp, n, ldx, out);
+    const int v = v4 ? 4 : 1;
+    auto go = [&](auto v_c, auto h_c, auto th_c) {
+        constexpr int TH = decltype(th_c)::value;
+        hipLaunchKernelGGL((k_act_prologue<decltype(v_c)::value, decltype(h_c)::value, TH>), dim3(T), dim3(TH), 0, st, x,
+                           x_res, res_out, rms_w, eps, div, x_up, clamp, n, ldx, out);
     };
-    if (v4) held ? go(std::integral_constant<int, 4>{}, std::true_type{}) : go(std::integral_constant<int, 4>{}, std::false_type{});
-    else held ? go(std::integral_constant<int, 1>{}, std::true_type{}) : go(std::integral_constant<int, 1>{}, std::false_type{});
+    auto rows = [&](auto v_c) {
+        if (n <= 256 * v) go(v_c, std::true_type{}, std::integral_constant<int, 256>{});
+        else if (n <= kProThreads * kProHeld * v) go(v_c, std::true_type{}, std::integral_constant<int, kProThreads>{});
+        else go(v_c, std::false_type{}, std::integral_constant<int, kProThreads>{});
+    };
+    if (v4) rows(std::integral_constant<int, 4>{});
+    else rows(std::integral_constant<int, 1>{});
     return hipGetLastError();
 }
 

@@ -221,11 +221,13 @@ def test_fused_silu_pair_batched(dev, orc, sem, R, C, B, mode):
     assert err < tol, K.last_error(dev.so)
 
 
-@pytest.mark.parametrize("C,ld,B", [(2880, 2881, 3), (17408, 17408, 9), (67584, 67584, 9), (5120, 5123, 9)])
+@pytest.mark.parametrize("C,ld,B", [(2880, 2881, 3), (17408, 17408, 9), (67584, 67584, 9), (5120, 5123, 9),
+                                    (1024, 1024, 9), (1056, 1056, 11), (256, 259, 10), (288, 291, 9), (32, 32, 130)])
 def test_fused_prologue_kernel_rows(dev, orc, C, ld, B):
     """The standalone prologue's forms: rows and strides that are no multiple of
-    four elements (scalar accesses), rows of several groups per thread, and rows
-    longer than its registers hold (scalar past 4096, vector past 16384)."""
+    four elements (scalar accesses), rows of several groups per thread, rows
+    longer than its registers hold (scalar past 4096, vector past 16384), and
+    short rows, which 256 threads take (scalar to 256, vector to 1024)."""
     import torch
     rng = np.random.default_rng(C + B)
     R, sem = 40, K.MXFP4
