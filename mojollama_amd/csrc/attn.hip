@@ -4,8 +4,9 @@
 // A decode step reads every cached K and V row once: the work is streaming
 // 2 * seq * n_kv_head * head_dim * 4 bytes, and what decides its rate is how
 // many of those bytes are in flight.  So the unit of work is one wave on one
-// 64-position chunk of one KV head, which requests its whole chunk before it
-// uses any of it and serves all n_head / n_kv_head query heads that share the
+// 64-position chunk of one KV head, which requests 64 elements of every K row
+// (the whole row up to head_dim 64) or a 64-element block of every V row before
+// it uses any of it and serves all n_head / n_kv_head query heads that share the
 // rows (GQA).  Both reference softmaxes need the maximum over all positions
 // before any weight (gqa_attention.c's exp_ps_simd is not an exponential, so
 // the online rescaling of flash decoding would not reproduce it), hence three

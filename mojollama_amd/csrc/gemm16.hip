@@ -1014,7 +1014,7 @@ __global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int 
     }
     if (TPR < 256 && row >= rows) return;
     const float *xr = x + (long)row * ldx;
-    const bool vec = ((uintptr_t)xr & 15) == 0;
+    const bool vec = ((uintptr_t)xr & 15) == 0;   // (and the prologue's vectors: 16-byte aligned, x's stride)
     const int nb = K / Q::EPS;
     // eight consecutive elements from k (a multiple of 8)
     auto ld8 = [&](int k, float (&v)[8]) __attribute__((always_inline)) {

@@ -61,7 +61,8 @@ struct mllm_gemv_args {
 };
 
 // moe_forward_omp's SiLU product (QK:2157-2164): the gate clamped to +-80,
-// then silu(g) * u.  Every kernel that forms it uses this one expression;
+// then silu(g) * u.  Every kernel that forms it uses this one expression, but the
+// grouped GEMMs' epilogue on the fp16 plane (silu16 in gemm16.hip, a few ulp from it);
 // clamp = false gives the unclamped form of moe_ffn and the dense FFN.
 __device__ __forceinline__ float mllm_silu_mul(float g, float u, bool clamp = true)
 {
